@@ -339,7 +339,7 @@ static void launch_xw_t(lh_handle* h, int want_cfl) {
   XW a{h->zu, h->zw, h->zv, h->zp, sizeof(TR) == 8 ? (const void*)h->twxw : (const void*)h->twxw32,
        h->dthdyu, h->scal, want_cfl, h->xraw_lc};
   const int nlev = h->dm.nyu - 2;
-  const long waves = (long)(h->dm.px / 2) * ((nlev + h->xraw_lc - 1) / h->xraw_lc);
+  const long waves = (long)(h->dm.pz / 2) * ((nlev + h->xraw_lc - 1) / h->xraw_lc);
   constexpr int W = XwWaves<TR>::value;
   const dim3 grid((unsigned)((waves + W - 1) / W)), block(64 * W);
   const size_t sh = xw_lds_bytes<W, TR>();
@@ -1096,7 +1096,7 @@ int lh_create(const lh_config* c, lh_handle** out) {
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)xibw_lds_bytes()));
       const int wpb = f64 ? XwWaves<double>::value : XwWaves<float>::value;
       if (h->xraw_lc <= 0)
-        h->xraw_lc = chunk_levels(dm.nyu - 2, (long)dm.px / 2, ncu * wpb, 4, 96, 1.0 / 3.0);
+        h->xraw_lc = chunk_levels(dm.nyu - 2, (long)dm.pz / 2, ncu * wpb, 4, 96, 1.0 / 3.0);
     }
     if (h->xraw_lc <= 0) h->xraw_lc = chunk_levels(dm.nyu - 2, dm.pz / 2, ncu * bx, 4, 64, 1.0);
     if (h->zasm_lc <= 0)

@@ -315,8 +315,8 @@ template <typename C> __device__ __forceinline__ void store_line(const C (&v)[9]
 }  // namespace xw
 
 struct XW {
-  const void *zu, *zw, *zv;      // Z slots [slot][576][193] (cx<TR>)
-  void* zp;                      // [6][level][288][2 * 193] packed row pairs (cx<TR>)
+  const void *zu, *zw, *zv;      // Z slots [slot][pz][193] (cx<TR>)
+  void* zp;                      // [6][level][pz / 2][2 * 193] packed row pairs (cx<TR>)
   const void* tw;                // xw::TWN twiddles (cx<TR>)
   const double* dthdyu;
   double* scal;
@@ -358,13 +358,13 @@ __global__ void __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(x
   C* buf = lds + xw::TWN + wv * (xw::LINE + 9 * 64);
   C* pk = buf + xw::LINE + t;                    // park line: slot s at pk[64 s]
   const int nlev = dm.nyu - 2;
-  const int npair = xw::N / 2;
+  const int npair = dm.pz / 2;
   const int item = blockIdx.x * WPB + wv;
   const int pair = item % npair, chunk = item / npair;
   const int l0 = chunk * a.lc;
   const int l1 = min(l0 + a.lc, nlev);
   if (l0 >= l1) return;
-  const size_t slot = (size_t)xw::N * xw::MX;
+  const size_t slot = (size_t)dm.pz * xw::MX;
   const size_t row = (size_t)pair * 2 * xw::MX;
   const C* zu = static_cast<const C*>(a.zu);
   const C* zw = static_cast<const C*>(a.zw);
