@@ -117,9 +117,10 @@ int lh_substep(lh_handle* h, int krk, double dt);
  *   lh_solve_u: RHS0_u1/u2/u3 (littleharsh.f90:166-168, with Nu_old from the other buffer
  *     and Nu_new from lh_nonlinear), the immersed boundaries and solveU/V/U
  *     (littleharsh.f90:173-175; tridLU_3D_IB.f90:50-359): u, v, w before the pressure step.
- *     RHS0 is formed inside the sweep, so it has no hook of its own.
+ *     RHS0 is formed inside the solve, so it has no hook of its own.
  *   lh_solve_p: meanflow_ctU when flag_ctpress = 0, solveP and v_corr
- *     (littleharsh.f90:178-188): v_corr is fused into the Poisson sweep. */
+ *     (littleharsh.f90:178-188).  lh_substep runs lh_solve_u's column part and this one in one
+ *     kernel, which keeps the velocities in registers in between. */
 int lh_nonlinear(lh_handle* h, int krk);
 int lh_solve_u(lh_handle* h, int krk, double dt);
 int lh_solve_p(lh_handle* h, int krk, double dt);
@@ -318,8 +319,8 @@ const char* lh_closure_last_error(const lh_closure* c);
 #define LH_K_ASM 3    /* forward z transforms of the products -> Nu       */
 #define LH_K_IBZ 4    /* canopy-plane z transforms                         */
 #define LH_K_XIB 5    /* canopy-plane x transforms + forcing               */
-#define LH_K_VEL 6    /* velocity Thomas sweeps                            */
-#define LH_K_PRES 7   /* pressure solve + v_corr                          */
+#define LH_K_VEL 6    /* column stage: velocity and pressure solves, v_corr */
+#define LH_K_PRES 7   /* (unused: the column stage is one class)          */
 #define LH_K_MISC 8   /* small kernels: LU factors, mean flow, scalars     */
 #define LH_K_RHS 9    /* RHS0 + nonlinear + rhs of the solves, per column  */
 #define LH_K_STEP 10  /* one replay of the captured RK3 step graph (mode 2) */

@@ -6,11 +6,11 @@
 //                (x transforms, six products, CFL max)
 //                -> k_zasm (A/B recombination, forward z transforms -> Nu_new)
 //   IB stage   : k_rhs_ib (rhs and Lu_y on canopy planes) -> k_zinv -> k_xpass_ib -> k_zfwd
-//   column     : k_prep (LU of the shared velocity matrices) -> k_vel_rhs (RHS0 + rhs of
-//                solveU/V on the fly, Thomas u, w, v)
-//                -> k_pres (constant-flow-rate correction, solveP, v_corr); these read the
-//                channel's parameters from a job table, so that a batch launches them once
-//                for all its members
+//   column     : k_prep (LU of the shared velocity matrices) -> k_col (RHS0 + rhs of solveU/V,
+//                the velocity solves, constant-flow-rate correction, solveP, v_corr; two
+//                one-thread-per-column kernels in mixed precision and for very tall channels); these
+//                read the channel's parameters from a job table, so that a batch launches them
+//                once for all its members
 // Statistics and spectra (lh_stats.hpp) run on request, outside the substep.
 // lh_step replays a captured HIP graph of three substeps (+ meanflow_ctP).
 #include <hip/hip_runtime.h>
@@ -29,6 +29,7 @@
 #include "lh_nl.hpp"
 #include "lh_xw.hpp"
 #include "lh_col.hpp"
+#include "lh_colf.hpp"
 #include "lh_stats.hpp"
 #include "lh_internal.hpp"
 
@@ -40,9 +41,7 @@ struct IbSets;
 // Default launch parameters (per handle; lh_autotune may change them):
 //   LH_XRAW_LC  levels per block of the sliding x pass (0: chosen per grid, see chunk_levels)
 //   LH_ZASM_LC  levels per block of the z assembly (0: chosen per grid)
-//   LH_COL_BS   threads per block of the canopy rhs kernel (one column per thread; the column
-//               stage itself runs 64 columns per block, which spread the 74k columns of the
-//               production grid evenly over the 256 CUs)
+//   LH_COL_BS   threads per block of the canopy rhs kernel (one column per thread)
 #ifndef LH_XRAW_LC
 #define LH_XRAW_LC 0
 #endif
@@ -137,9 +136,6 @@ struct lh_handle {
   int zasm_lc = LH_ZASM_LC;
   int col_bs = LH_COL_BS;
   int xplan = 0, zplan = 0;     // FFT plan of the x and z lengths (Plan<n, v>)
-  // rows per step of the velocity sweep: 1 on large grids (fewer registers, more resident
-  // waves), kVelUSmall when few columns leave the sweeps latency-bound (set at creation)
-  int vel_u = 1;
   // per-kernel timing (direct issue, an event pair per launch) or, with timing_steps, one
   // event pair around each replay of the captured step graph
   bool timing = false;
@@ -257,15 +253,6 @@ static bool supported_len(int n) {
 #ifndef LH_COL_U
 #define LH_COL_U 8
 #endif
-#ifndef LH_VEL_U
-#define LH_VEL_U 1
-#endif
-// Grids of at most kVelSmallCols spectral columns run the velocity sweep kVelUSmall rows per
-// step: with one thread per column too few waves are resident to hide each row's loads
-// (96x145x96: 1.37 -> 1.24 ms per step; 64x97x64: 0.89 -> 0.82 ms; the pressure sweep's
-// unroll and the block size change nothing there).
-constexpr int kVelSmallCols = 16384;
-constexpr int kVelUSmall = 4;
 template <int N, int V> constexpr int zlines() {
   return N >= 384 ? LH_ZLINES_LONG : (Plan<N, V>::T >= 8 ? 16 : 32);
 }
@@ -523,10 +510,17 @@ static void nu_buffers(const lh_handle* h, int krk, double2* nw[3], double2* ol[
   nw[0] = wb ? h->nb1 : h->nu1; nw[1] = wb ? h->nb2 : h->nu2; nw[2] = wb ? h->nb3 : h->nu3;
   ol[0] = wb ? h->nu1 : h->nb1; ol[1] = wb ? h->nu2 : h->nb2; ol[2] = wb ? h->nu3 : h->nb3;
 }
+static int col_kind(const lh_handle* h);
+static CTU make_ctu(const lh_handle* h, int krk) {
+  const Dims& dm = h->dm;
+  return CTU{h->u1, h->scal, h->ctwork, h->dyu2i, h->yv, h->gw[0], h->gw[1], h->rk[3 + krk] / dm.re,
+             h->rk[12 + krk], dm.ny, dm.d, dm.ncol};
+}
 static PREP make_prep(const lh_handle* h, int krk) {
   const Dims& dm = h->dm;
   const double bre = h->rk[3 + krk] / dm.re;
-  return PREP{h->dyu2i, h->dyv2i, h->scal, h->ayu, h->ayv, h->gw[0], h->gw[1], bre, dm.nyu, dm.nyv};
+  return PREP{h->dyu2i, h->dyv2i, h->scal, h->ayu, h->ayv, h->gw[0], h->gw[1], bre, dm.nyu, dm.nyv,
+              h->flag_ctpress == 0 && col_kind(h) > 0 ? 1 : 0, make_ctu(h, krk)};
 }
 static RHS make_rhs(const lh_handle* h, int krk) {
   const Dims& dm = h->dm;
@@ -551,7 +545,7 @@ static RHS make_rhs(const lh_handle* h, int krk) {
 }
 static COL make_col(const lh_handle* h, int krk) {
   const Dims& dm = h->dm;
-  const double aR = h->rk[krk], bR = h->rk[3 + krk], dR = h->rk[12 + krk];
+  const double aR = h->rk[krk], bR = h->rk[3 + krk];
   COL a{};
   a.r1 = h->r1; a.r2 = h->r2; a.r3 = h->r3;
   a.u1 = h->u1; a.u2 = h->u2; a.u3 = h->u3; a.p = h->p; a.psi = h->psi;
@@ -560,18 +554,14 @@ static COL make_col(const lh_handle* h, int krk) {
   a.dthdyu = h->dthdyu; a.dthdyv = h->dthdyv; a.k1x = h->k1x; a.k1z = h->k1z;
   a.scal = h->scal; a.ab = aR + bR; a.gw0 = h->gw[0]; a.gw1 = h->gw[1];
   a.ctu = h->flag_ctpress == 0 ? 1 : 0;
-  a.ct = CTU{h->u1, h->scal, h->ctwork, h->dyu2i, h->yv, h->gw[0], h->gw[1], bR / dm.re, dR, dm.ny,
-             dm.d, dm.ncol};
+  a.ct = make_ctu(h, krk);
   return a;
 }
 
-// The column stage (k_prep, the velocity sweeps, the pressure step, the flow rate) runs from
-// job tables: a job holds one channel's parameters for one substep, and block b of a launch
-// works on channel colmap[b], columns (b - blk0) * 64 + lane.  A single channel launches
-// them with its own table (one job per substep); a batch launches them once for all its
-// members.  Small channels have a few thousand spectral columns, so one channel's column
-// kernels fill a few percent of the device for the time of their sequential sweep over the
-// planes; launched together, the members' sweeps run side by side.  Both launch the same
+// The column stage (k_prep, k_col, the flow rate) runs from job tables: a job holds one
+// channel's parameters for one substep, and block b of a launch works on channel colmap[b],
+// columns from (b - blk0) times the columns per block.  A single channel launches them with its own table (one
+// job per substep); a batch launches them once for all its members.  Both launch the same
 // kernels, so a batch member computes exactly what the channel computes alone.
 struct ColJob {
   RHS ra;
@@ -579,17 +569,39 @@ struct ColJob {
   PREP prep;
   Dims dm;
   const double* yv;
-  int vel_u;        // rows per step of the member's velocity sweep
-  int blk0;         // first block of the member in the launches of its sweep kernels
+  int blk0;         // first block of the member in the launches of its column kernel
   int flowrate;     // flag_ctpress == 1: flowrateRe after the step
 };
-constexpr int kMultiCols = 64;
-__global__ void __launch_bounds__(64) k_prep(const ColJob* __restrict__ jobs) {
-  prep_body(jobs[blockIdx.x].prep, threadIdx.x);
+__global__ void __launch_bounds__(192) k_prep(const ColJob* __restrict__ jobs) {
+  const PREP& a = jobs[blockIdx.x].prep;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (w < 2 || a.ctu) prep_body(a, w, threadIdx.x & 63);
 }
-// one kernel per row unroll of the velocity sweep (their register needs differ: 72 VGPRs at
-// one row per step, 150 at four); a batch orders its members' blocks by unroll and launches
-// each variant over its range, blocks boff, boff + 1, ...
+// The shapes of k_col: R levels per thread, CB columns per block, most threads per block, and
+// whether a thread loads all its rows up front (see col_kind for the choice).  256 registers and
+// no spills each, so that a CU holds 8 waves: with 9 levels and 16 columns one block spans 288
+// levels and reads 256 contiguous bytes of a plane at a time.
+template <int KIND> struct ColShape;
+template <> struct ColShape<1> { static constexpr int R = 4, CB = 8, T = 512; static constexpr bool PRE = true; };
+template <> struct ColShape<2> { static constexpr int R = 9, CB = 16, T = 512; static constexpr bool PRE = false; };
+template <> struct ColShape<3> { static constexpr int R = 9, CB = 8, T = 512; static constexpr bool PRE = false; };
+// rows of a component loaded together when not all are (9 at a time spill)
+constexpr int kColRows = 3;
+template <int KIND, int MODE>
+__global__ void __launch_bounds__(ColShape<KIND>::T) __attribute__((amdgpu_waves_per_eu(2)))
+    k_col(const ColJob* __restrict__ jobs, const int* __restrict__ colmap, int boff) {
+  using S = ColShape<KIND>;
+  extern __shared__ char smem_raw[];
+  const int b = blockIdx.x + boff;
+  const ColJob& J = jobs[colmap[b]];
+  const Dims dm = J.dm;
+  const RHS ra = J.ra;
+  const COL ca = J.ca;
+  colf_block<S::R, S::CB, S::PRE ? S::R : kColRows, S::PRE, MODE>(ra, ca, dm, J.yv, (b - J.blk0) * S::CB, smem_raw);
+}
+// The sweeps with one thread per column, 64 columns per block.  One kernel per row unroll of the
+// velocity sweep (their register needs differ: 72 VGPRs at one row per step, 150 at four).
+constexpr int kMultiCols = 64;
 template <int U>
 __global__ void __launch_bounds__(kMultiCols) k_vel_rhs(const ColJob* __restrict__ jobs,
                                                           const int* __restrict__ colmap, int boff) {
@@ -602,10 +614,11 @@ __global__ void __launch_bounds__(kMultiCols) k_vel_rhs(const ColJob* __restrict
   vel_column<U>(ra, dm, c, blockIdx.y, J.ca.ayu, J.ca.ayv);
 }
 __global__ void __launch_bounds__(kMultiCols) k_pres(const ColJob* __restrict__ jobs,
-                                                           const int* __restrict__ colmap) {
-  const ColJob& J = jobs[colmap[blockIdx.x]];
+                                                           const int* __restrict__ colmap, int boff) {
+  const int b = blockIdx.x + boff;
+  const ColJob& J = jobs[colmap[b]];
   const Dims dm = J.dm;
-  const int c = (blockIdx.x - J.blk0) * kMultiCols + threadIdx.x;
+  const int c = (b - J.blk0) * kMultiCols + threadIdx.x;
   if (c >= dm.ncol) return;
   const COL ca = J.ca;
   pres_column<LH_COL_U>(ca, dm, c);
@@ -646,12 +659,91 @@ static ColJob make_job(const lh_handle* h, int krk, int blk0) {
   J.prep = make_prep(h, krk);
   J.dm = h->dm;
   J.yv = h->yv;
-  J.vel_u = h->vel_u;
   J.blk0 = blk0;
   J.flowrate = h->flag_ctpress == 1 ? 1 : 0;
   return J;
 }
-static int col_blocks(const lh_handle* h) { return (h->dm.ncol + kMultiCols - 1) / kMultiCols; }
+// The column kernel of a channel, by its columns and levels (np), with the times of a launch of
+// the column stage (before: the two one-thread-per-column kernels it replaces):
+//   1  4 levels x 8 columns, all rows loaded up front: grids of at most kColSmall columns, whose
+//      few blocks leave each thread's chain of memory latencies as the time (544 columns, 41
+//      planes: 14 us, kind 2 19 us, before 47 us; 2112 columns, 97 planes: 25 us, kind 2 24 us)
+//   2  9 levels x 16 columns: 4704 columns, 145 planes 41 us (kind 1 69 us, before 169 us); 74112
+//      columns, 289 planes 1.19 ms (before 2.13 ms): 5.0 GB at 4.2 TB/s, a device copy's 4.7 TB/s
+//   3  9 levels x 8 columns: more than 288 levels (74112 columns, 289 planes: 1.26 ms)
+//   0, -1  one thread per column (k_vel_rhs, k_pres): more than 576 levels, and the mixed-precision
+//      mode.  There the FP32 stage turns a last-bit difference of the state into one as large as
+//      its own rounding errors (one flipped rounding of a plane's mean re-rounds the plane), so
+//      the order of these operations, which k_col changes, is part of that mode's results:
+//      with k_col they would move by 4e-5 in p, as far as they are from FP64.  -1: at most
+//      kVelSmallCols columns, whose velocity sweep takes 4 rows per step: too few waves are
+//      resident there to hide each row's loads.
+constexpr int kColSmall = 1600, kVelSmallCols = 16384;
+template <int KIND> static bool col_fits(const Dims& dm) {
+  using S = ColShape<KIND>;
+  return (dm.nyp + S::R - 1) / S::R * S::CB <= S::T;
+}
+static int col_kind(const lh_handle* h) {
+  const Dims& dm = h->dm;
+  if (h->prec == LH_PREC_FP64) {
+    if (dm.ncol <= kColSmall && col_fits<1>(dm)) return 1;
+    if (col_fits<2>(dm)) return 2;
+    if (col_fits<3>(dm)) return 3;
+  }
+  return dm.ncol <= kVelSmallCols ? -1 : 0;
+}
+static int col_blocks(const lh_handle* h) {
+  const int kind = col_kind(h);
+  const int cb = kind == 1 ? ColShape<1>::CB : (kind == 2 ? ColShape<2>::CB : (kind == 3 ? ColShape<3>::CB : kMultiCols));
+  return (h->dm.ncol + cb - 1) / cb;
+}
+static int col_chunks(const lh_handle* h) {
+  const int kind = col_kind(h);
+  const int r = kind == 1 ? ColShape<1>::R : ColShape<2>::R;
+  return kind > 0 ? (h->dm.nyp + r - 1) / r : 0;
+}
+// launches the column kernel of a kind over blocks boff .. boff + nb - 1 of a job table, whose
+// channels have at most nc chunks per column and nyu planes
+template <int KIND>
+static void launch_col_t(hipStream_t st, const ColJob* jobs, const int* map, int boff, int nb, int nc, int nyu, int mode) {
+  using S = ColShape<KIND>;
+  const size_t sh = colf_lds_bytes(nyu, nc, S::R, S::CB);
+  const dim3 g(nb), t(nc * S::CB);
+  if (mode == kColAll) hipLaunchKernelGGL((k_col<KIND, kColAll>), g, t, sh, st, jobs, map, boff);
+  else if (mode == kColVel) hipLaunchKernelGGL((k_col<KIND, kColVel>), g, t, sh, st, jobs, map, boff);
+  else hipLaunchKernelGGL((k_col<KIND, kColPres>), g, t, sh, st, jobs, map, boff);
+}
+static void launch_col(int kind, hipStream_t st, const ColJob* jobs, const int* map, int boff, int nb, int nc, int nyu,
+                       int mode) {
+  switch (kind) {
+    case 1: launch_col_t<1>(st, jobs, map, boff, nb, nc, nyu, mode); break;
+    case 2: launch_col_t<2>(st, jobs, map, boff, nb, nc, nyu, mode); break;
+    case 3: launch_col_t<3>(st, jobs, map, boff, nb, nc, nyu, mode); break;
+    default:
+      if (mode & kColVel) {
+        if (kind < 0) hipLaunchKernelGGL(k_vel_rhs<4>, dim3(nb, 3), dim3(kMultiCols), 0, st, jobs, map, boff);
+        else hipLaunchKernelGGL(k_vel_rhs<1>, dim3(nb, 3), dim3(kMultiCols), 0, st, jobs, map, boff);
+      }
+      if (mode & kColPres) hipLaunchKernelGGL(k_pres, dim3(nb), dim3(kMultiCols), 0, st, jobs, map, boff);
+  }
+}
+template <int KIND> static hipError_t attr_col_t() {
+  const void* const f[3] = {(const void*)k_col<KIND, kColAll>, (const void*)k_col<KIND, kColVel>,
+                            (const void*)k_col<KIND, kColPres>};
+  for (const void* k : f) {
+    const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+static hipError_t attr_col(const lh_handle* h) {
+  switch (col_kind(h)) {
+    case 1: return attr_col_t<1>();
+    case 2: return attr_col_t<2>();
+    case 3: return attr_col_t<3>();
+    default: return hipSuccess;
+  }
+}
 
 // ---- the canopy stage from job tables (channels whose transform lengths are all <= 144)
 // A channel of that size runs its canopy stage from tables, alone or in a batch; within a
@@ -859,7 +951,7 @@ static void issue_substep(lh_handle* h, int krk /*0-based*/, bool cfl_mode, int 
   auto fork_prep = [&]() {
     (void)hipEventRecord(h->ev_fork, h->st);
     (void)hipStreamWaitEvent(h->side, h->ev_fork, 0);
-    hipLaunchKernelGGL(k_prep, dim3(1), dim3(64), 0, h->side, (const ColJob*)h->coljobs + krk);
+    hipLaunchKernelGGL(k_prep, dim3(1), dim3(192), 0, h->side, (const ColJob*)h->coljobs + krk);
     (void)hipEventRecord(h->ev_join, h->side);
   };
   const bool late = krk == 0 && cfl_mode;
@@ -978,28 +1070,17 @@ static void issue_substep(lh_handle* h, int krk /*0-based*/, bool cfl_mode, int 
   // ---- column stage
   if (side)
     (void)hipStreamWaitEvent(h->st, h->ev_join, 0);
-  else if (stages & kStageVelCol)
+  else if (stages & (kStageVelCol | kStagePres))
     TIMED(h, LH_K_MISC, 0.0,
-          hipLaunchKernelGGL(k_prep, dim3(1), dim3(64), 0, h->st, (const ColJob*)h->coljobs + krk));
+          hipLaunchKernelGGL(k_prep, dim3(1), dim3(192), 0, h->st, (const ColJob*)h->coljobs + krk));
   {
     const ColJob* jk = h->coljobs + krk;
-    const int nb = col_blocks(h);
-    // in: rhs u, w, v, p, LU factors (8 B each); out: u, w, v, p
-    const double by = spl * (2.0 * nuvw + 2.0 * dm.nyp) + 3.0 * 8.0 * dm.ncol * (double)dm.nyp;
-    // in: u, p, Nu_old, Nu_new (rhs on canopy planes); eliminated rows out and back; out: u
-    if (stages & kStageVelCol)
-    TIMED(h, LH_K_VEL, spl * (7.0 * nuvw), {
-      if (h->vel_u == kVelUSmall)
-        hipLaunchKernelGGL(k_vel_rhs<kVelUSmall>, dim3(nb, 3), dim3(kMultiCols), 0, h->st, jk,
-                           (const int*)h->colmap, 0);
-      else
-        hipLaunchKernelGGL(k_vel_rhs<LH_VEL_U>, dim3(nb, 3), dim3(kMultiCols), 0, h->st, jk,
-                           (const int*)h->colmap, 0);
-    });
-    if (stages & kStagePres)
-    TIMED(h, LH_K_PRES, by - 2.0 * nuvw * spl + 2.0 * nuvw * spl,
-          hipLaunchKernelGGL(k_pres, dim3(nb), dim3(kMultiCols), 0, h->st, jk,
-                             (const int*)h->colmap));
+    const int mode = ((stages & kStageVelCol) ? kColVel : 0) | ((stages & kStagePres) ? kColPres : 0);
+    // in: u, w, v, Nu_old, Nu_new (or the canopy rhs), p, the Poisson factors; out: u, w, v, p
+    const double by = spl * ((krk == 0 ? 3.0 : 4.0) * nuvw + 2.5 * dm.nyp);
+    if (mode)
+      TIMED(h, LH_K_VEL, by, launch_col(col_kind(h), h->st, jk, (const int*)h->colmap, 0, col_blocks(h),
+                                        col_chunks(h), dm.nyu, mode));
   }
 }
 
@@ -1035,7 +1116,6 @@ int lh_create(const lh_config* c, lh_handle** out) {
   Dims& dm = h->dm;
   dm.nx = c->nx; dm.nz = c->nz; dm.px = c->px; dm.pz = c->pz;
   dm.mx = c->nx / 2 + 1; dm.ncol = dm.mx * c->nz;
-  h->vel_u = dm.ncol <= kVelSmallCols ? kVelUSmall : LH_VEL_U;
   dm.ny = c->ny; dm.d = c->dsty;
   dm.nyu = c->ny + 2 * c->dsty + 1; dm.nyv = c->ny + 2 * c->dsty; dm.nyp = c->ny + 2 * c->dsty - 1;
   dm.dxi = c->px * c->alp / (2.0 * M_PI);
@@ -1129,7 +1209,8 @@ int lh_create(const lh_config* c, lh_handle** out) {
   }
   // state and work
   HIPCHK(h, dalloc(&h->u1, nu)); HIPCHK(h, dalloc(&h->u3, nu)); HIPCHK(h, dalloc(&h->u2, nv));
-  HIPCHK(h, dalloc(&h->p, np)); HIPCHK(h, dalloc(&h->psi, np));
+  HIPCHK(h, dalloc(&h->p, np));
+  if (col_kind(h) <= 0) HIPCHK(h, dalloc(&h->psi, np));     // k_pres's eliminated rows
   HIPCHK(h, dalloc(&h->nu1, nu)); HIPCHK(h, dalloc(&h->nu3, nu)); HIPCHK(h, dalloc(&h->nu2, nv));
   HIPCHK(h, dalloc(&h->nb1, nu)); HIPCHK(h, dalloc(&h->nb3, nu)); HIPCHK(h, dalloc(&h->nb2, nv));
   HIPCHK(h, dalloc(&h->r1, nu)); HIPCHK(h, dalloc(&h->r3, nu)); HIPCHK(h, dalloc(&h->r2, nv));
@@ -1294,6 +1375,7 @@ int lh_create(const lh_config* c, lh_handle** out) {
     std::vector<ColJob> jobs;
     for (int k = 0; k < 3; ++k) jobs.push_back(make_job(h, k, 0));
     const std::vector<int> map(col_blocks(h), 0);
+    HIPCHK(h, attr_col(h));
     HIPCHK(h, hipMalloc((void**)&h->coljobs, jobs.size() * sizeof(ColJob)));
     HIPCHK(h, hipMalloc((void**)&h->colmap, map.size() * sizeof(int)));
     HIPCHK(h, hipMemcpy(h->coljobs, jobs.data(), jobs.size() * sizeof(ColJob), hipMemcpyHostToDevice));
@@ -1848,19 +1930,26 @@ int lh_batch_step_cfl(lh_batch* b, double cfl) {
     // the device, where the graph's launches read them)
     const int n = (int)b->hs.size();
     std::vector<ColJob> jobs(3 * (size_t)n);
-    // blocks of the members with the small-grid sweep (kVelUSmall rows per step) first
+    // block ranges of the members that share a column kernel
+    struct Range { int kind, boff, nb, nc, nyu; };
+    std::vector<Range> ranges;
     std::vector<int> colmap;
-    int nblk = 0, nsmall = 0;
-    for (int pass = 0; pass < 2; ++pass)
+    int nblk = 0;
+    for (int kind : {1, 2, 3, 0, -1}) {
+      Range g{kind, nblk, 0, 0, 0};
       for (int i = 0; i < n; ++i) {
         lh_handle* h = b->hs[i];
-        if ((h->vel_u == kVelUSmall) != (pass == 0)) continue;
+        if (col_kind(h) != kind) continue;
         for (int k = 0; k < 3; ++k) jobs[(size_t)k * n + i] = make_job(h, k, nblk);
         const int nb = col_blocks(h);
         colmap.insert(colmap.end(), nb, i);
         nblk += nb;
-        if (pass == 0) nsmall = nblk;
+        g.nb += nb;
+        g.nc = std::max(g.nc, col_chunks(h));
+        g.nyu = std::max(g.nyu, h->dm.nyu);
       }
+      if (g.nb > 0) ranges.push_back(g);
+    }
     if (b->jobs) { (void)hipFree(b->jobs); b->jobs = nullptr; }
     if (b->colmap) { (void)hipFree(b->colmap); b->colmap = nullptr; }
     if (!chk(hipMalloc((void**)&b->jobs, jobs.size() * sizeof(ColJob)), "job table") ||
@@ -1906,15 +1995,9 @@ int lh_batch_step_cfl(lh_batch* b, double cfl) {
       if (k == 0) hipLaunchKernelGGL(k_jobs_cfl_dt, dim3(sb), dim3(64), 0, b->master, (const ColJob*)b->jobs, n);
       b->ib.launch(k, b->master);
       const ColJob* jk = b->jobs + (size_t)k * n;
-      hipLaunchKernelGGL(k_prep, dim3(n), dim3(64), 0, b->master, jk);
-      if (nsmall > 0)
-        hipLaunchKernelGGL(k_vel_rhs<kVelUSmall>, dim3(nsmall, 3), dim3(kMultiCols), 0, b->master, jk,
-                           (const int*)b->colmap, 0);
-      if (nblk > nsmall)
-        hipLaunchKernelGGL(k_vel_rhs<LH_VEL_U>, dim3(nblk - nsmall, 3), dim3(kMultiCols), 0, b->master,
-                           jk, (const int*)b->colmap, nsmall);
-      hipLaunchKernelGGL(k_pres, dim3(nblk), dim3(kMultiCols), 0, b->master, jk,
-                         (const int*)b->colmap);
+      hipLaunchKernelGGL(k_prep, dim3(n), dim3(192), 0, b->master, jk);
+      for (const Range& g : ranges)
+        launch_col(g.kind, b->master, jk, (const int*)b->colmap, g.boff, g.nb, g.nc, g.nyu, kColAll);
     }
     hipLaunchKernelGGL(k_flowrate, dim3(n), dim3(256), 0, b->master, (const ColJob*)b->jobs);
     hipLaunchKernelGGL(k_jobs_scalars, dim3(sb), dim3(64), 0, b->master, (const ColJob*)b->jobs, n, b->dscal);

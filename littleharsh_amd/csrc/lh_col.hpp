@@ -1,11 +1,12 @@
-// lh_col.hpp -- column stage of the RK3 substep: one thread per spectral column (kx, kz)
-// builds the rhs of solveU/solveV and runs the velocity Thomas sweeps of LUsolU/LUsolV
-// (tridLU_3D_IB.f90:106-116, 179-189),
-// the constant-flow-rate correction of the (0,0) column when enabled (flowrate_corr,
-// littleharsh.f90:453-485), solveP with LUsolP (littleharsh.f90:557-612,
-// tridLU_3D_IB.f90:362-396) and v_corr (littleharsh.f90:826-929).  Consecutive columns
-// sit on consecutive lanes, so every row access is coalesced; rows are processed U at a
-// time with all loads issued before the dependent recurrence.
+// lh_col.hpp -- column stage of the RK3 substep with one thread per spectral column (kx, kz), for
+// channels too tall for the kernel of lh_colf.hpp and for the mixed-precision mode, and the rhs
+// of the canopy planes: builds the
+// rhs of solveU/solveV and runs the velocity Thomas sweeps of LUsolU/LUsolV
+// (tridLU_3D_IB.f90:106-116, 179-189), the constant-flow-rate correction of the (0,0) column when
+// enabled (flowrate_corr, littleharsh.f90:453-485), solveP with LUsolP (littleharsh.f90:557-612,
+// tridLU_3D_IB.f90:362-396) and v_corr (littleharsh.f90:826-929).  Consecutive columns sit on
+// consecutive lanes, so every row access is coalesced; rows are processed U at a time with all
+// loads issued before the dependent recurrence.
 #pragma once
 #include "lh_kernels.hpp"
 
@@ -70,9 +71,9 @@ __device__ void ctu_column(const CTU& a) {
 //   Lu  = dy2i(1,s) u(s-1) + (k2x + k2z + dy2i(2,s)) u(s) + dy2i(3,s) u(s+1)
 //   du  = aRK/Re Lu - cRK Nu_old - dRK grad p [- dRK mpgx on the (0,0) u mode] - gRK Nu_new
 //   rhs = (u + dt du) / axz
-// The velocity sweeps (k_vel) evaluate it on the fly; the canopy planes, which the
-// immersed-boundary stage rewrites in physical space first, get it from k_rhs_ib together
-// with Lu_y on the tip planes.
+// The column kernels evaluate it on the fly; the canopy planes, which the immersed-boundary
+// stage rewrites in physical space first, get it from k_rhs_ib together with Lu_y on the tip
+// planes.
 struct RHS {
   double2 *u1, *u2, *u3;
   const double2* p;

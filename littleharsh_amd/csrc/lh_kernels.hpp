@@ -498,59 +498,107 @@ __device__ __forceinline__ double2 dim(double k, double2 a) { return d2(-k * a.y
 // ------------------------------------------------------------------------------------
 // Column stage
 // ------------------------------------------------------------------------------------
+// flowrate_corr + LUsol0 (littleharsh.f90:453-485; tridLU_3D_IB.f90:398-424, 573-599,
+// 686-703) on the (0,0) column
+struct CTU {
+  double2* u1;
+  double* scal;
+  double* work;            // u11(0..ny), qx1, then ny + 1 values of scratch
+  const double *dyu2i, *yv;
+  double gw0, gw1, bre, dR;
+  int ny, d, ncol;
+};
+
 // LU_build + LU_dec of the shared velocity matrices (tridLU_3D_IB.f90:427-493, 601-640)
 struct PREP {
   const double *dyu2i, *dyv2i, *scal;
   double *ayu, *ayv;     // [rows][3]
   double gw0, gw1, bre;
   int nyu, nyv;
+  int ctu;               // the response of the mean flow too (flag_ctpress == 0)
+  CTU ct;
 };
 
-// LU_build + LU_dec of the two shared y matrices (tridLU_3D_IB.f90:427-493, 601-640), one
-// thread per grid.  The recurrence runs in registers (the previous row's scaled upper
-// entry is the only carried value) with the operations in the order of LU_dec.
-__device__ __forceinline__ void prep_body(const PREP& a, int t) {
-  if (t > 1) return;
-  const int nj = t == 0 ? a.nyu : a.nyv;
-  const gptr<const double> dd = gp(t == 0 ? a.dyu2i : a.dyv2i);
-  const gptr<double> ay = gp(t == 0 ? a.ayu : a.ayv);
-  const double beta = a.bre * gp(a.scal)[S_DT];
-  // row 0: (0, 1, gw(1)) on the u grid, Dirichlet (0, 1, 0) on the v grid
-  double up = t == 0 ? a.gw0 : 0.0;
-  double di = 1.0 / 1.0;
-  ay[0] = 0.0;
-  ay[1] = di;
-  for (int r = 1; r < nj; ++r) {
-    double lo, dg, upr;
-    if (r < nj - 1) {
-      lo = -beta * dd[3 * r + 0];
-      dg = 1.0 - beta * dd[3 * r + 1];
-      upr = -beta * dd[3 * r + 2];
-    } else {                      // last row: (gw(2), 1, 0) on the u grid, (0, 1, 0) on v
-      lo = t == 0 ? a.gw1 : 0.0;
-      dg = 1.0;
-      upr = 0.0;
-    }
-    const double a3 = up * di;    // upper of row r-1 scaled by its 1/diag
-    ay[3 * (r - 1) + 2] = a3;
-    di = 1.0 / (dg - lo * a3);
-    ay[3 * r + 0] = lo;
-    ay[3 * r + 1] = di;
-    up = upr;
-  }
-  ay[3 * (nj - 1) + 2] = up;
+__device__ __forceinline__ double lane_of(double v, int i) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), i),
+                          __builtin_amdgcn_readlane(__double2loint(v), i));
 }
 
-// flowrate_corr + LUsol0 (littleharsh.f90:453-485; tridLU_3D_IB.f90:398-424, 573-599,
-// 686-703) on the (0,0) column; one thread.
-struct CTU {
-  double2* u1;
-  double* scal;
-  double* work;            // 4*(ny+1)
-  const double *dyu2i, *yv;
-  double gw0, gw1, bre, dR;
-  int ny, d, ncol;
-};
+// LU_build + LU_dec, one wave per system: wave 0 the u grid, wave 1 the v grid, wave 2 the mean
+// flow's response to a unit pressure gradient (LU_build0, LU_dec0, LUsol0 on the rows between
+// the post tips).  A lane builds one row of a tile of 64; every lane then runs the recurrence
+// of the tile from the rows' lanes (v_readlane) with the operations in the order of LU_dec, so
+// that a row costs its division chain and no memory latency (289 planes: 92 us with a load
+// per row, one thread).
+__device__ __forceinline__ void prep_body(const PREP& a, int w, int l) {
+  const double beta = a.bre * gp(a.scal)[S_DT];
+  const int d = w == 2 ? a.ct.d : 0;
+  const int nj = w == 0 ? a.nyu : (w == 1 ? a.nyv : a.ct.ny + 1);
+  const gptr<const double> dd = gp(w == 1 ? a.dyv2i : a.dyu2i) + 3 * d;
+  const double gw0 = w == 1 ? 0.0 : a.gw0, gw1 = w == 1 ? 0.0 : a.gw1;
+  const gptr<double> ay = gp(w == 1 ? a.ayv : a.ayu);
+  const gptr<double> u11 = gp(a.ct.work), m3 = u11 + (a.ct.ny + 2);
+  const double bdt = -a.ct.dR * gp(a.scal)[S_DT];
+  double a3 = 0.0, y = 0.0;                  // scaled upper and eliminated rhs of the row before
+  for (int t0 = 0; t0 < nj; t0 += 64) {
+    const int r = t0 + l;
+    // boundary rows: (0, 1, gw(1)) and (gw(2), 1, 0) on the u grid, (0, 1, 0) on the v grid
+    double lo = 0.0, dg = 1.0, up = 0.0;
+    if (r == 0) {
+      up = gw0;
+    } else if (r < nj - 1) {
+      lo = -beta * dd[3 * r + 0];
+      dg = 1.0 - beta * dd[3 * r + 1];
+      up = -beta * dd[3 * r + 2];
+    } else if (r == nj - 1) {
+      lo = gw1;
+    }
+    const double rhs = r > 0 && r < nj - 1 ? bdt : 0.0;
+    double di = 0.0, a3r = 0.0, yr = 0.0;
+    const int nt = min(64, nj - t0);
+    for (int i = 0; i < nt; ++i) {
+      const double li = lane_of(lo, i);
+      const double dii = 1.0 / (lane_of(dg, i) - li * a3);
+      if (w == 2) y = (lane_of(rhs, i) - li * y) * dii;
+      a3 = lane_of(up, i) * dii;
+      if (l == i) {
+        di = dii;
+        a3r = a3;
+        yr = y;
+      }
+    }
+    if (r < nj) {
+      if (w < 2) {
+        ay[3 * r + 0] = lo;
+        ay[3 * r + 1] = di;
+        ay[3 * r + 2] = r == nj - 1 ? up : a3r;
+      } else {
+        u11[r] = yr;
+        m3[r] = a3r;
+      }
+    }
+  }
+  if (w < 2) return;
+  // back substitution, then the flow rate of the response: flowrateRe(Qx1, u11) declares its
+  // dummy u(1:nn+2) while u11 is (0:nn+2) (littleharsh.f90:443 vs 472-474), so that u(j) is
+  // u11(j-1) there
+  const int n = a.ct.ny;
+  const gptr<const double> yv = gp(a.ct.yv);
+  double x = 0.0, q = 0.0;
+  for (int t0 = (n / 64) * 64; t0 >= 0; t0 -= 64) {
+    const int r = t0 + l;
+    const double yr = r <= n ? u11[r] : 0.0, ar = r < n ? m3[r] : 0.0;
+    double xr = 0.0;
+    for (int i = min(63, n - t0); i >= 0; --i) {
+      x = lane_of(yr, i) - lane_of(ar, i) * x;
+      if (l == i) xr = x;
+    }
+    if (r <= n) u11[r] = xr;
+    if (r <= n - 2) q += (yv[r + 1 + d] - yv[r + d]) * xr;
+  }
+  for (int off = 32; off > 0; off >>= 1) q += __shfl_down(q, off, 64);
+  if (l == 0) u11[n + 1] = q;
+}
 
 // Row r of the Poisson operator D G + k^2 of one column (LU_buildP, tridLU_3D_IB.f90:497-571):
 // lower lo, diagonal dg and upper up; p row r <-> plane j = r - d + 1, u/v slot r + 1.  Row 0
