@@ -31,6 +31,7 @@
 #include "lh_col.hpp"
 #include "lh_colf.hpp"
 #include "lh_stats.hpp"
+#include "lh_xfer.hpp"
 #include "lh_internal.hpp"
 
 using namespace lh;
@@ -138,6 +139,7 @@ struct lh_handle {
   int xplan = 0, zplan = 0;     // FFT plan of the x and z lengths (Plan<n, v>)
   // per-kernel timing (direct issue, an event pair per launch) or, with timing_steps, one
   // event pair around each replay of the captured step graph
+  bool staged = false;          // holds a share of the process's pinned buffers (lh_xfer.hpp)
   bool timing = false;
   bool timing_steps = false;
   // batches the handle belongs to: while any, the handle's own graphs keep k_prep on its
@@ -1134,6 +1136,8 @@ int lh_create(const lh_config* c, lh_handle** out) {
     if (c->tip_v[t] < -dm.d + 1 || c->tip_v[t] > dm.ny + dm.d - 2) return bad("tip_v out of range");
   }
   *out = h;
+  host_stage().retain();
+  h->staged = true;
   HIPCHK(h, hipGetDevice(&h->dev));
   HIPCHK(h, hipStreamCreate(&h->st));
   HIPCHK(h, hipStreamCreate(&h->side));
@@ -1421,89 +1425,81 @@ int lh_destroy(lh_handle* h) {
   if (h->side) hipStreamDestroy(h->side);
   if (h->ev_fork) (void)hipEventDestroy(h->ev_fork);
   if (h->ev_join) (void)hipEventDestroy(h->ev_join);
+  if (h->staged) host_stage().release();
   delete h;
   return LH_OK;
 }
 
-// reference layout f(j, column) <-> device [plane][column]
-static int upload_field(lh_handle* h, double2* dst, const double* src, int nj) {
+// Fields between the host's layout f(j, column) and the device's [plane][column], staged in zp
+// (free between substeps; it holds the four state fields and the five spectra).
+static int xfer_fields(lh_handle* h, XferFields& fs, int nf, bool up, bool cplx) {
   const int ncol = h->dm.ncol;
-  std::vector<double2> t((size_t)nj * ncol);
-  const double2* s = reinterpret_cast<const double2*>(src);
-  for (int c = 0; c < ncol; ++c)
-    for (int j = 0; j < nj; ++j) t[(size_t)j * ncol + c] = s[(size_t)c * nj + j];
-  HIPCHK(h, hipMemcpy(dst, t.data(), t.size() * sizeof(double2), hipMemcpyHostToDevice));
+  const size_t el = cplx ? sizeof(double2) : sizeof(double);
+  HIPCHK(h, hipStreamSynchronize(h->st));
+  size_t off = 0;
+  int most = 0;
+  for (int i = 0; i < nf; ++i) {
+    XferField& f = fs.f[i];
+    f.stage = off;
+    if (!f.host) {
+      f.n = f.nj = 0;                                  // no blocks
+      continue;
+    }
+    off += (size_t)f.n * ncol * el;
+    most = std::max(most, up ? f.nj : f.n);
+  }
+  if (off == 0) return LH_OK;
+  char* const stage = static_cast<char*>(h->zp);
+  const dim3 grid((ncol + kXT - 1) / kXT, (most + kXT - 1) / kXT, nf), block(kXT * 8);
+  if (up) HIPCHK(h, xfer_bytes(true, h->dev, h->st, stage, fs, nf, ncol, el));
+  if (cplx && up) hipLaunchKernelGGL((k_xfer<double2, true>), grid, block, 0, h->st, fs, stage, ncol);
+  else if (cplx) hipLaunchKernelGGL((k_xfer<double2, false>), grid, block, 0, h->st, fs, stage, ncol);
+  else hipLaunchKernelGGL((k_xfer<double, false>), grid, block, 0, h->st, fs, stage, ncol);
+  HIPCHK(h, hipGetLastError());
+  if (up) HIPCHK(h, hipStreamSynchronize(h->st));
+  else HIPCHK(h, xfer_bytes(false, h->dev, h->st, stage, fs, nf, ncol, el));
   return LH_OK;
 }
-static int download_field(lh_handle* h, double* dst, const double2* src, int nj) {
-  const int ncol = h->dm.ncol;
-  std::vector<double2> t((size_t)nj * ncol);
-  HIPCHK(h, hipMemcpy(t.data(), src, t.size() * sizeof(double2), hipMemcpyDeviceToHost));
-  double2* d = reinterpret_cast<double2*>(dst);
-  for (int c = 0; c < ncol; ++c)
-    for (int j = 0; j < nj; ++j) d[(size_t)c * nj + j] = t[(size_t)j * ncol + c];
-  return LH_OK;
+static XferField whole(double2* dev, const double* host, int nj) {
+  return XferField{dev, const_cast<double*>(host), 0, nj, 0, nj};
+}
+// Nu in the reference's allocation range jlim(1)+1 : jlim(2)-1 (littleharsh.f90:122-124)
+static XferField inner(double2* dev, const double* host, int nj) {
+  return XferField{dev, const_cast<double*>(host), 0, nj, 1, nj - 2};
 }
 
 int lh_set_state(lh_handle* h, const double* u1, const double* u2, const double* u3, const double* p) {
   if (!h) return LH_ERR_ARG;
-  HIPCHK(h, hipStreamSynchronize(h->st));
-  int r;
-  if (u1 && (r = upload_field(h, h->u1, u1, h->dm.nyu))) return r;
-  if (u2 && (r = upload_field(h, h->u2, u2, h->dm.nyv))) return r;
-  if (u3 && (r = upload_field(h, h->u3, u3, h->dm.nyu))) return r;
-  if (p && (r = upload_field(h, h->p, p, h->dm.nyp))) return r;
-  return LH_OK;
+  const Dims& dm = h->dm;
+  XferFields fs{{whole(h->u1, u1, dm.nyu), whole(h->u2, u2, dm.nyv), whole(h->u3, u3, dm.nyu), whole(h->p, p, dm.nyp)}};
+  return xfer_fields(h, fs, 4, true, true);
 }
 
 int lh_get_state(lh_handle* h, double* u1, double* u2, double* u3, double* p) {
   if (!h) return LH_ERR_ARG;
-  HIPCHK(h, hipStreamSynchronize(h->st));
-  int r;
-  if (u1 && (r = download_field(h, u1, h->u1, h->dm.nyu))) return r;
-  if (u2 && (r = download_field(h, u2, h->u2, h->dm.nyv))) return r;
-  if (u3 && (r = download_field(h, u3, h->u3, h->dm.nyu))) return r;
-  if (p && (r = download_field(h, p, h->p, h->dm.nyp))) return r;
-  return LH_OK;
+  const Dims& dm = h->dm;
+  XferFields fs{{whole(h->u1, u1, dm.nyu), whole(h->u2, u2, dm.nyv), whole(h->u3, u3, dm.nyu), whole(h->p, p, dm.nyp)}};
+  return xfer_fields(h, fs, 4, false, true);
 }
 
-// Nu in the reference's allocation range jlim(1)+1 : jlim(2)-1 (littleharsh.f90:122-124)
-static int xfer_nl(lh_handle* h, double2* dev, double* host, int nj, bool up) {
-  const int ncol = h->dm.ncol;
-  std::vector<double2> t((size_t)nj * ncol);
-  if (!up) HIPCHK(h, hipMemcpy(t.data(), dev, t.size() * 16, hipMemcpyDeviceToHost));
-  double2* hh = reinterpret_cast<double2*>(host);
-  for (int c = 0; c < ncol; ++c)
-    for (int r = 0; r < nj - 2; ++r) {
-      if (up) t[(size_t)(r + 1) * ncol + c] = hh[(size_t)c * (nj - 2) + r];
-      else hh[(size_t)c * (nj - 2) + r] = t[(size_t)(r + 1) * ncol + c];
-    }
-  if (up) HIPCHK(h, hipMemcpy(dev, t.data(), t.size() * 16, hipMemcpyHostToDevice));
-  return LH_OK;
+static int xfer_nl(lh_handle* h, double2* a, double2* b, double2* c, const double* n1, const double* n2,
+                   const double* n3, bool up) {
+  const Dims& dm = h->dm;
+  XferFields fs{{inner(a, n1, dm.nyu), inner(b, n2, dm.nyv), inner(c, n3, dm.nyu)}};
+  return xfer_fields(h, fs, 3, up, true);
 }
 
 int lh_set_nonlinear(lh_handle* h, const double* n1, const double* n2, const double* n3) {
   if (!h) return LH_ERR_ARG;
-  HIPCHK(h, hipStreamSynchronize(h->st));
-  int r;
   // both buffers: the next substep reads whichever its parity selects
-  for (int b = 0; b < 2; ++b) {
-    if (n1 && (r = xfer_nl(h, b ? h->nb1 : h->nu1, (double*)n1, h->dm.nyu, true))) return r;
-    if (n2 && (r = xfer_nl(h, b ? h->nb2 : h->nu2, (double*)n2, h->dm.nyv, true))) return r;
-    if (n3 && (r = xfer_nl(h, b ? h->nb3 : h->nu3, (double*)n3, h->dm.nyu, true))) return r;
-  }
-  return LH_OK;
+  const int r = xfer_nl(h, h->nu1, h->nu2, h->nu3, n1, n2, n3, true);
+  return r ? r : xfer_nl(h, h->nb1, h->nb2, h->nb3, n1, n2, n3, true);
 }
 
 int lh_get_nonlinear(lh_handle* h, double* n1, double* n2, double* n3) {
   if (!h) return LH_ERR_ARG;
-  HIPCHK(h, hipStreamSynchronize(h->st));
-  int r;
-  const bool b = h->nu_last == 1;
-  if (n1 && (r = xfer_nl(h, b ? h->nb1 : h->nu1, n1, h->dm.nyu, false))) return r;
-  if (n2 && (r = xfer_nl(h, b ? h->nb2 : h->nu2, n2, h->dm.nyv, false))) return r;
-  if (n3 && (r = xfer_nl(h, b ? h->nb3 : h->nu3, n3, h->dm.nyu, false))) return r;
-  return LH_OK;
+  if (h->nu_last == 1) return xfer_nl(h, h->nb1, h->nb2, h->nb3, n1, n2, n3, false);
+  return xfer_nl(h, h->nu1, h->nu2, h->nu3, n1, n2, n3, false);
 }
 
 // one stage of substep kRK on the handle's stream, synchronous at return
@@ -1697,13 +1693,11 @@ int lh_set_forcing(lh_handle* h, const double* f1, const double* f2, const doubl
   if (!h->fo1) {
     HIPCHK(h, dalloc(&h->fo1, nu)); HIPCHK(h, dalloc(&h->fo3, nu)); HIPCHK(h, dalloc(&h->fo2, nv));
   }
-  // a null field is zero; the ghost planes of every field stay zero
-  std::vector<double> zero(2 * nu, 0.0);
-  int r;
-  if ((r = xfer_nl(h, h->fo1, (double*)(f1 ? f1 : zero.data()), h->dm.nyu, true))) return r;
-  if ((r = xfer_nl(h, h->fo2, (double*)(f2 ? f2 : zero.data()), h->dm.nyv, true))) return r;
-  if ((r = xfer_nl(h, h->fo3, (double*)(f3 ? f3 : zero.data()), h->dm.nyu, true))) return r;
-  return LH_OK;
+  // a null field is zero, as are the ghost planes of every field
+  if (!f1) HIPCHK(h, hipMemset(h->fo1, 0, nu * sizeof(double2)));
+  if (!f2) HIPCHK(h, hipMemset(h->fo2, 0, nv * sizeof(double2)));
+  if (!f3) HIPCHK(h, hipMemset(h->fo3, 0, nu * sizeof(double2)));
+  return xfer_nl(h, h->fo1, h->fo2, h->fo3, f1, f2, f3, true);
 }
 
 }  // extern "C"
@@ -1738,11 +1732,7 @@ int lh_get_forcing(lh_handle* h, double* f1, double* f2, double* f3) {
   if (!h) return LH_ERR_ARG;
   HIPCHK(h, hipStreamSynchronize(h->st));
   if (!h->fo1) return fail(h, LH_ERR_ARG, "lh_get_forcing: no forcing has been set");
-  int r;
-  if (f1 && (r = xfer_nl(h, h->fo1, f1, h->dm.nyu, false))) return r;
-  if (f2 && (r = xfer_nl(h, h->fo2, f2, h->dm.nyv, false))) return r;
-  if (f3 && (r = xfer_nl(h, h->fo3, f3, h->dm.nyu, false))) return r;
-  return LH_OK;
+  return xfer_nl(h, h->fo1, h->fo2, h->fo3, f1, f2, f3, false);
 }
 
 int lh_get_launch(lh_handle* h, int* xraw_lc, int* zasm_lc, int* col_bs) {
@@ -2207,18 +2197,15 @@ int lh_spectra_read(lh_handle* h, double* out, int reset) {
   if (!h || !out) return LH_ERR_ARG;
   const Dims& dm = h->dm;
   const size_t pl = (size_t)dm.nyu * dm.ncol;
-  HIPCHK(h, hipStreamSynchronize(h->st));
   if (!h->sp_acc) {
     memset(out, 0, 5 * pl * sizeof(double));
     return LH_OK;
   }
-  std::vector<double> t(5 * pl);
-  HIPCHK(h, hipMemcpy(t.data(), h->sp_acc, t.size() * sizeof(double), hipMemcpyDeviceToHost));
   // device [f][slot][column] -> sp(j, column), j fastest, each array ncol x nyu
-  for (int f = 0; f < 5; ++f)
-    for (int c = 0; c < dm.ncol; ++c)
-      for (int s = 0; s < dm.nyu; ++s)
-        out[f * pl + (size_t)c * dm.nyu + s] = t[f * pl + (size_t)s * dm.ncol + c];
+  XferFields fs{};
+  for (int f = 0; f < 5; ++f) fs.f[f] = XferField{h->sp_acc + f * pl, out + f * pl, 0, dm.nyu, 0, dm.nyu};
+  const int r = xfer_fields(h, fs, 5, false, false);
+  if (r) return r;
   if (reset) HIPCHK(h, hipMemset(h->sp_acc, 0, 5 * pl * sizeof(double)));
   return LH_OK;
 }

@@ -72,10 +72,10 @@ class Channel:
 
     def get_state(self):
         s = self.s
-        u = np.zeros((s.ncol, s.nyu), complex)
-        v = np.zeros((s.ncol, s.nyv), complex)
-        w = np.zeros((s.ncol, s.nyu), complex)
-        p = np.zeros((s.ncol, s.nyp), complex)
+        u = np.empty((s.ncol, s.nyu), complex)
+        v = np.empty((s.ncol, s.nyv), complex)
+        w = np.empty((s.ncol, s.nyu), complex)
+        p = np.empty((s.ncol, s.nyp), complex)
         self._chk(self._lib.lh_get_state(self._h, _p(u), _p(v), _p(w), _p(p)), "lh_get_state")
         return u, v, w, p
 
@@ -93,9 +93,9 @@ class Channel:
 
     def get_nonlinear(self):
         s = self.s
-        n1 = np.zeros((s.ncol, s.nyu - 2), complex)
-        n2 = np.zeros((s.ncol, s.nyv - 2), complex)
-        n3 = np.zeros((s.ncol, s.nyu - 2), complex)
+        n1 = np.empty((s.ncol, s.nyu - 2), complex)
+        n2 = np.empty((s.ncol, s.nyv - 2), complex)
+        n3 = np.empty((s.ncol, s.nyu - 2), complex)
         self._chk(self._lib.lh_get_nonlinear(self._h, _p(n1), _p(n2), _p(n3)), "lh_get_nonlinear")
         return n1, n2, n3
 
@@ -112,9 +112,9 @@ class Channel:
 
     def get_forcing(self):
         s = self.s
-        f1 = np.zeros((s.ncol, s.nyu - 2), complex)
-        f2 = np.zeros((s.ncol, s.nyv - 2), complex)
-        f3 = np.zeros((s.ncol, s.nyu - 2), complex)
+        f1 = np.empty((s.ncol, s.nyu - 2), complex)
+        f2 = np.empty((s.ncol, s.nyv - 2), complex)
+        f3 = np.empty((s.ncol, s.nyu - 2), complex)
         self._chk(self._lib.lh_get_forcing(self._h, _p(f1), _p(f2), _p(f3)), "lh_get_forcing")
         return f1, f2, f3
 
@@ -171,7 +171,7 @@ class Channel:
 
     def spectra(self, reset: bool = False):
         """(5, ncol, nyu): U, V, W, UV, P in the reference layout sp(j, column)."""
-        a = np.zeros((5, self.s.ncol, self.s.nyu))
+        a = np.empty((5, self.s.ncol, self.s.nyu))
         self._chk(self._lib.lh_spectra_read(self._h, _p(a), 1 if reset else 0), "lh_spectra_read")
         return a
 
