@@ -75,10 +75,6 @@ struct lh_handle {
   std::string err;
   int dev = 0;
   hipStream_t st = nullptr;
-  // side stream for the LU of the velocity matrices (k_prep), which needs only dt: it runs
-  // beside the nonlinear stage, forked and joined by the two events
-  hipStream_t side = nullptr;
-  hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   Dims dm{};
   int prec = LH_PREC_FP64;
   int flag_ctpress = 1;
@@ -142,12 +138,10 @@ struct lh_handle {
   bool staged = false;          // holds a share of the process's pinned buffers (lh_xfer.hpp)
   bool timing = false;
   bool timing_steps = false;
-  // batches the handle belongs to: while any, the handle's own graphs keep k_prep on its
-  // stream (a batch runs the column stage of all its members itself; a side branch per
-  // substep and instance, 48 x 3 cross-stream joins per step, serialised the instances)
+  // batches the handle belongs to (lh_destroy refuses while any)
   int in_batch = 0;
   // bumped whenever the captured graphs are dropped (launch parameters, forcing switched on
-  // or off, batch membership): a batch re-captures when a member's generation changed
+  // or off): a batch re-captures when a member's generation changed
   unsigned gen = 0;
   std::vector<hipEvent_t> evpool;
   size_t evnext = 0;
@@ -371,7 +365,7 @@ template <int PZ, typename TR, int V>
 static void launch_zasm_t(lh_handle* h, const ZASM& a, const void* tw) {
   constexpr int L = kZasmCols;
   const int nlev = h->dm.nyu - 2;
-  dim3 grid(a.nib * ((nlev + a.lc - 1) / a.lc) * 3);
+  dim3 grid(a.nib * ((nlev + a.lc - 1) / a.lc) * 3 + (a.prep ? kPrepBlocks : 0));
   const size_t sh = zasm_lds<PZ, TR, V>();
   hipLaunchKernelGGL((k_zasm<PZ, L, TR, V>), grid, dim3(2 * L * Plan<PZ, V>::T), sh, h->st, a, h->dm,
                      (const cx<TR>*)tw);
@@ -500,9 +494,16 @@ constexpr int kStageNLz = 1, kStageIBr = 2, kStagePres = 4, kStageVelCol = 8, kS
 // with a stage: the caller clears the CFL maximum and forms the time step of a CFL step
 // (a batch does both for all its members in one launch each)
 constexpr int kCallerCfl = 512;
+// with the assembly alone: it forms the LU of the velocity matrices too (dt is known)
+constexpr int kAsmPrep = 1024;
 constexpr int kStageNL = kStageNLz | kStageNLx | kStageNLa;
 constexpr int kStageIB = kStageIBr | kStageIBz | kStageIBx | kStageIBf;
 constexpr int kStageVel = kStageIB | kStageVelCol, kStageAll = kStageNL | kStageVel | kStagePres;
+
+// whether the LU of the velocity matrices is formed in the assembly's launch
+static bool prep_in_asm(int stages) {
+  return (stages & kAsmPrep) || ((stages & kStageNLa) && (stages & kStageVelCol));
+}
 
 // parameters of the column stage of substep krk (0-based); the batch builds them for every
 // member and launches the column kernels of all members at once
@@ -946,18 +947,6 @@ static void issue_substep(lh_handle* h, int krk /*0-based*/, bool cfl_mode, int 
   const double zsl = zel * dm.pz * dm.mx;                    // bytes per Z slot
   const double spl = 16.0 * dm.ncol;                         // bytes per spectral plane
   const double nuvw = 2.0 * dm.nyu + dm.nyv;                 // u, w, v planes
-  // k_prep needs only dt: in graph and direct issue it runs on the side stream beside the
-  // nonlinear stage (timing mode and batch members keep it in line); at kRK = 1 of a CFL
-  // step dt comes from the first x pass, so it forks after k_cfl_dt
-  const bool side = !h->timing && h->in_batch == 0 && stages == kStageAll;
-  auto fork_prep = [&]() {
-    (void)hipEventRecord(h->ev_fork, h->st);
-    (void)hipStreamWaitEvent(h->side, h->ev_fork, 0);
-    hipLaunchKernelGGL(k_prep, dim3(1), dim3(192), 0, h->side, (const ColJob*)h->coljobs + krk);
-    (void)hipEventRecord(h->ev_join, h->side);
-  };
-  const bool late = krk == 0 && cfl_mode;
-  if (side && !late) fork_prep();
   double2 *nw[3], *ol[3];
   nu_buffers(h, krk, nw, ol);
   const bool wb = (krk % 2) == 1;
@@ -988,7 +977,6 @@ static void issue_substep(lh_handle* h, int krk /*0-based*/, bool cfl_mode, int 
   }
   if (krk == 0 && cfl_mode && !(stages & kCallerCfl))
     TIMED(h, LH_K_MISC, 0.0, hipLaunchKernelGGL(k_cfl_dt, dim3(1), dim3(1), 0, h->st, h->scal));
-  if (side && late) fork_prep();
   }
   if (stages & kStageNLa) {
   h->nu_last = wb ? 1 : 0;
@@ -999,6 +987,7 @@ static void issue_substep(lh_handle* h, int krk /*0-based*/, bool cfl_mode, int 
     a.dthdyu = h->dthdyu; a.dthdyv = h->dthdyv; a.k1x = h->k1x; a.k1z = h->k1z;
     a.nib = (dm.mx + kZasmCols - 1) / kZasmCols;
     a.lc = h->zasm_lc;
+    a.prep = prep_in_asm(stages) ? &h->coljobs[krk].prep : nullptr;
     // in: six product Z rows per level; out: Nu_new
     const double by = 6.0 * nlev * zsl + spl * (2.0 * nlev + (nlev - 1));
     TIMED(h, LH_K_ASM, by, {
@@ -1070,9 +1059,7 @@ static void issue_substep(lh_handle* h, int krk /*0-based*/, bool cfl_mode, int 
           launch_zfwd(h, fj, 3, h->nibu > h->nibv ? h->nibu : h->nibv, true));
   }
   // ---- column stage
-  if (side)
-    (void)hipStreamWaitEvent(h->st, h->ev_join, 0);
-  else if (stages & (kStageVelCol | kStagePres))
+  if ((stages & (kStageVelCol | kStagePres)) && !prep_in_asm(stages))
     TIMED(h, LH_K_MISC, 0.0,
           hipLaunchKernelGGL(k_prep, dim3(1), dim3(192), 0, h->st, (const ColJob*)h->coljobs + krk));
   {
@@ -1140,9 +1127,6 @@ int lh_create(const lh_config* c, lh_handle** out) {
   h->staged = true;
   HIPCHK(h, hipGetDevice(&h->dev));
   HIPCHK(h, hipStreamCreate(&h->st));
-  HIPCHK(h, hipStreamCreate(&h->side));
-  HIPCHK(h, hipEventCreateWithFlags(&h->ev_fork, hipEventDisableTiming));
-  HIPCHK(h, hipEventCreateWithFlags(&h->ev_join, hipEventDisableTiming));
   {
     int dummy = 0;
     for (int v = 0; v < plans_of_len(c->pz); ++v) {
@@ -1401,7 +1385,6 @@ int lh_destroy(lh_handle* h) {
   // a batch keeps pointers to its members: it must be destroyed first
   if (h->in_batch > 0) return fail(h, LH_ERR_ARG, "lh_destroy: the handle belongs to a batch; destroy the batch first");
   if (h->st) hipStreamSynchronize(h->st);
-  if (h->side) hipStreamSynchronize(h->side);
   for (auto& g : h->gexec)
     if (g) (void)hipGraphExecDestroy(g);
   for (auto e : h->evpool) (void)hipEventDestroy(e);
@@ -1422,9 +1405,6 @@ int lh_destroy(lh_handle* h) {
   if (h->twx64) hipFree(h->twx64);
   if (h->twz64) hipFree(h->twz64);
   if (h->st) hipStreamDestroy(h->st);
-  if (h->side) hipStreamDestroy(h->side);
-  if (h->ev_fork) (void)hipEventDestroy(h->ev_fork);
-  if (h->ev_join) (void)hipEventDestroy(h->ev_join);
   if (h->staged) host_stage().release();
   delete h;
   return LH_OK;
@@ -1893,7 +1873,6 @@ int lh_batch_create(int n, lh_handle* const* hs, lh_batch** out) {
     }
   for (auto* h : b->hs) {
     h->in_batch += 1;
-    drop_graphs(h);                                 // captured with the side branch
   }
   b->joined = true;
   *out = b;
@@ -1974,7 +1953,9 @@ int lh_batch_step_cfl(lh_batch* b, double cfl) {
       for (int ph : phases)
         for (int i = 0; i < n && ok; ++i) {
           lh_handle* h = b->hs[i];
-          if (!((ph & kStageIB) && ib_jobs(h))) issue_substep(h, k, true, ph | (small_channel(h) ? kCallerCfl : 0));
+          if (!((ph & kStageIB) && ib_jobs(h))) 
+            issue_substep(h, k, true, ph | (small_channel(h) ? kCallerCfl : 0) |
+                                          (k > 0 && ph == kStageNLa ? kAsmPrep : 0));
         }
       for (int i = 0; i < n && ok; ++i) {
         lh_handle* h = b->hs[i];
@@ -1985,7 +1966,8 @@ int lh_batch_step_cfl(lh_batch* b, double cfl) {
       if (k == 0) hipLaunchKernelGGL(k_jobs_cfl_dt, dim3(sb), dim3(64), 0, b->master, (const ColJob*)b->jobs, n);
       b->ib.launch(k, b->master);
       const ColJob* jk = b->jobs + (size_t)k * n;
-      hipLaunchKernelGGL(k_prep, dim3(n), dim3(192), 0, b->master, jk);
+      // (the time step of the first substep comes after the join)
+      if (k == 0) hipLaunchKernelGGL(k_prep, dim3(n), dim3(192), 0, b->master, jk);
       for (const Range& g : ranges)
         launch_col(g.kind, b->master, jk, (const int*)b->colmap, g.boff, g.nb, g.nc, g.nyu, kColAll);
     }
@@ -2028,7 +2010,6 @@ int lh_batch_destroy(lh_batch* b) {
   if (b->joined)
     for (auto* h : b->hs) {
       h->in_batch -= 1;
-      drop_graphs(h);                               // captured with k_prep in line
     }
   if (b->g) (void)hipGraphExecDestroy(b->g);
   if (b->jobs) (void)hipFree(b->jobs);

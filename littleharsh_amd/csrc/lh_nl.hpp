@@ -262,7 +262,13 @@ struct ZASM {
   const double *dthdyu, *dthdyv, *k1x, *k1z;
   int nib;                                   // column blocks
   int lc;                                    // levels per block
+  // the LU of the velocity matrices for this substep's column stage, or null: it needs only dt,
+  // so three extra blocks of this launch form it (kPrepBlocks) beside the assembly, whose time
+  // covers the row-by-row recurrence; as a kernel of its own on a side stream its fork and join
+  // cost 15 us a substep
+  const PREP* prep;
 };
+constexpr int kPrepBlocks = 3;
 
 // twiddle table of the z assembly's transforms
 template <int PZ, typename C, int V = 0>
@@ -295,9 +301,17 @@ __global__ void __launch_bounds__((2 * L * Plan<PZ, V>::T))
   C* lds = reinterpret_cast<C*>(smem_raw);
   const int tid = threadIdx.x;
   const int nlev = dm.nyu - 2;
-  // XCD-aware remap of the linear block id (8 XCDs, round-robin dispatch)
-  const int nblk = gridDim.x;
   int bid = blockIdx.x;
+  if (a.prep) {
+    // the first blocks: one system each, on the block's first wave
+    if (bid < kPrepBlocks) {
+      if (tid < 64 && (bid < 2 || a.prep->ctu)) prep_body(*a.prep, bid, tid);
+      return;
+    }
+    bid -= kPrepBlocks;
+  }
+  // XCD-aware remap of the linear block id (8 XCDs, round-robin dispatch)
+  const int nblk = gridDim.x - (a.prep ? kPrepBlocks : 0);
   const int per = nblk / 8;
   if (bid < per * 8) bid = (bid % 8) * per + bid / 8;
   const int nch = (nlev + a.lc - 1) / a.lc;
