@@ -71,6 +71,7 @@ static int chunk_levels(int nlev, long colblocks, int ncu, int lo, int hi, doubl
 #define LH_COL_BS 64
 #endif
 
+constexpr int kHioIn = S_NSCAL;
 struct lh_handle {
   std::string err;
   int dev = 0;
@@ -87,6 +88,9 @@ struct lh_handle {
          *dyv2i = nullptr;
   double *k1x = nullptr, *k2x = nullptr, *k1z = nullptr, *k2z = nullptr;
   double* scal = nullptr;
+  // pinned host memory the device reads and writes (a slot of lh_xfer.hpp's): the scalars after a
+  // step, then the caller's value for the next one (kHioIn)
+  double* hio = nullptr;
   // state
   double2 *u1 = nullptr, *u2 = nullptr, *u3 = nullptr, *p = nullptr;
   // nonlinear terms, two buffers: substeps 1 and 3 write A and read B, substep 2 the reverse
@@ -135,7 +139,6 @@ struct lh_handle {
   int xplan = 0, zplan = 0;     // FFT plan of the x and z lengths (Plan<n, v>)
   // per-kernel timing (direct issue, an event pair per launch) or, with timing_steps, one
   // event pair around each replay of the captured step graph
-  bool staged = false;          // holds a share of the process's pinned buffers (lh_xfer.hpp)
   bool timing = false;
   bool timing_steps = false;
   // batches the handle belongs to (lh_destroy refuses while any)
@@ -206,7 +209,7 @@ static int fail(lh_handle* h, int code, const std::string& msg) {
 // littleharsh.f90:323-352).  The first x pass of every step takes the CFL maximum of the
 // state at the start of the step with a reduction that keeps NaN, so a non-finite value
 // anywhere in u, v or w shows there.  With need_dt the device CFL time step must also be
-// finite and positive.  Reads back the device scalars into s.
+// finite and positive.  s: the device scalars.
 static int check_scalars(lh_handle* h, bool need_dt, const double* s) {
   char msg[160];
   if (!std::isfinite(s[S_CFLMAX])) {
@@ -219,10 +222,6 @@ static int check_scalars(lh_handle* h, bool need_dt, const double* s) {
     return fail(h, LH_ERR_NUMERIC, msg);
   }
   return LH_OK;
-}
-static int numeric_check(lh_handle* h, bool need_dt, double* s) {
-  HIPCHK(h, hipMemcpy(s, h->scal, S_NSCAL * sizeof(double), hipMemcpyDeviceToHost));
-  return check_scalars(h, need_dt, s);
 }
 
 template <typename T>
@@ -496,6 +495,8 @@ constexpr int kStageNLz = 1, kStageIBr = 2, kStagePres = 4, kStageVelCol = 8, kS
 constexpr int kCallerCfl = 512;
 // with the assembly alone: it forms the LU of the velocity matrices too (dt is known)
 constexpr int kAsmPrep = 1024;
+// with every stage: the caller has cleared the CFL maximum (k_step_begin)
+constexpr int kBegun = 2048;
 constexpr int kStageNL = kStageNLz | kStageNLx | kStageNLa;
 constexpr int kStageIB = kStageIBr | kStageIBz | kStageIBx | kStageIBf;
 constexpr int kStageVel = kStageIB | kStageVelCol, kStageAll = kStageNL | kStageVel | kStagePres;
@@ -574,11 +575,12 @@ struct ColJob {
   const double* yv;
   int blk0;         // first block of the member in the launches of its column kernel
   int flowrate;     // flag_ctpress == 1: flowrateRe after the step
+  double* hout;     // pinned host copy of the scalars (null in a batch's table)
 };
 __global__ void __launch_bounds__(192) k_prep(const ColJob* __restrict__ jobs) {
   const PREP& a = jobs[blockIdx.x].prep;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  if (w < 2 || a.ctu) prep_body(a, w, threadIdx.x & 63);
+  if (w < 2 || a.ctu) prep_body(a, w, threadIdx.x & 63, gp(a.scal)[S_DT]);
 }
 // The shapes of k_col: R levels per thread, CB columns per block, most threads per block, and
 // whether a thread loads all its rows up front (see col_kind for the choice).  256 registers and
@@ -629,8 +631,9 @@ __global__ void __launch_bounds__(kMultiCols) k_pres(const ColJob* __restrict__ 
 __global__ void __launch_bounds__(256) k_flowrate(const ColJob* __restrict__ jobs) {
   __shared__ double part[256];
   const ColJob& J = jobs[blockIdx.x];
-  if (!J.flowrate) return;
-  flowrate_body(J.ca.u1, J.yv, J.ca.scal, J.dm.ny, J.dm.d, J.dm.ncol, part);
+  if (J.flowrate) flowrate_body(J.ca.u1, J.yv, J.ca.scal, J.dm.ny, J.dm.d, J.dm.ncol, part);
+  if (J.hout && threadIdx.x < S_NSCAL)
+    J.hout[threadIdx.x] = J.flowrate && threadIdx.x == S_QX ? part[0] : gp(J.ca.scal)[threadIdx.x];
 }
 // The scalars of the n channels of a job table, one thread per channel: the set-up of a CFL
 // step (the CFL number, and the maximum cleared for the x pass to accumulate), its time
@@ -655,7 +658,7 @@ __global__ void k_jobs_scalars(const ColJob* __restrict__ jobs, int n, double* _
   for (int q = 0; q < S_NSCAL; ++q) out[(size_t)i * S_NSCAL + q] = s[q];
 }
 
-static ColJob make_job(const lh_handle* h, int krk, int blk0) {
+static ColJob make_job(const lh_handle* h, int krk, int blk0, double* hout) {
   ColJob J;
   J.ra = make_rhs(h, krk);
   J.ca = make_col(h, krk);
@@ -664,6 +667,7 @@ static ColJob make_job(const lh_handle* h, int krk, int blk0) {
   J.yv = h->yv;
   J.blk0 = blk0;
   J.flowrate = h->flag_ctpress == 1 ? 1 : 0;
+  J.hout = hout;
   return J;
 }
 // The column kernel of a channel, by its columns and levels (np), with the times of a launch of
@@ -960,7 +964,7 @@ static void issue_substep(lh_handle* h, int krk /*0-based*/, bool cfl_mode, int 
     TIMED(h, LH_K_ZINV, nuvw * (spl + zsl), launch_zinv(h, jobs, 3, dm.nyu, false));
   }
   if (stages & kStageNLx) {
-  if (krk == 0 && !(stages & kCallerCfl))
+  if (krk == 0 && !(stages & (kCallerCfl | kBegun)))
     TIMED(h, LH_K_MISC, 0.0,
           hipLaunchKernelGGL(k_set_scalar, dim3(1), dim3(1), 0, h->st, h->scal, (int)S_CFLMAX, 0.0));
   {
@@ -975,7 +979,7 @@ static void issue_substep(lh_handle* h, int krk /*0-based*/, bool cfl_mode, int 
       }
     });
   }
-  if (krk == 0 && cfl_mode && !(stages & kCallerCfl))
+  if (krk == 0 && cfl_mode && !(stages & kCallerCfl) && !prep_in_asm(stages))
     TIMED(h, LH_K_MISC, 0.0, hipLaunchKernelGGL(k_cfl_dt, dim3(1), dim3(1), 0, h->st, h->scal));
   }
   if (stages & kStageNLa) {
@@ -988,6 +992,7 @@ static void issue_substep(lh_handle* h, int krk /*0-based*/, bool cfl_mode, int 
     a.nib = (dm.mx + kZasmCols - 1) / kZasmCols;
     a.lc = h->zasm_lc;
     a.prep = prep_in_asm(stages) ? &h->coljobs[krk].prep : nullptr;
+    a.cfl = krk == 0 && cfl_mode ? h->scal : nullptr;      // (used with prep only)
     // in: six product Z rows per level; out: Nu_new
     const double by = 6.0 * nlev * zsl + spl * (2.0 * nlev + (nlev - 1));
     TIMED(h, LH_K_ASM, by, {
@@ -1073,11 +1078,14 @@ static void issue_substep(lh_handle* h, int krk /*0-based*/, bool cfl_mode, int 
   }
 }
 
+// one step: the time step or the CFL number from hio[kHioIn], the scalars to hio at the end
 static void issue_step(lh_handle* h, bool cfl_mode) {
-  for (int k = 0; k < 3; ++k) issue_substep(h, k, cfl_mode);
-  if (h->flag_ctpress == 1)
-    TIMED(h, LH_K_MISC, 0.0,
-          hipLaunchKernelGGL(k_flowrate, dim3(1), dim3(256), 0, h->st, (const ColJob*)h->coljobs));
+  TIMED(h, LH_K_MISC, 0.0,
+        hipLaunchKernelGGL(k_step_begin, dim3(1), dim3(64), 0, h->st, h->scal, (const double*)h->hio + kHioIn,
+                           cfl_mode ? (int)S_CFL : (int)S_DT));
+  for (int k = 0; k < 3; ++k) issue_substep(h, k, cfl_mode, kStageAll | kBegun);
+  TIMED(h, LH_K_MISC, 0.0,
+        hipLaunchKernelGGL(k_flowrate, dim3(1), dim3(256), 0, h->st, (const ColJob*)h->coljobs));
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1123,8 +1131,9 @@ int lh_create(const lh_config* c, lh_handle** out) {
     if (c->tip_v[t] < -dm.d + 1 || c->tip_v[t] > dm.ny + dm.d - 2) return bad("tip_v out of range");
   }
   *out = h;
-  host_stage().retain();
-  h->staged = true;
+  static_assert(kHioIn < HostStage::kSlot, "scalars and the step's value fit a slot");
+  h->hio = host_stage().retain();
+  if (!h->hio) return fail(h, LH_ERR_HIP, "pinned host memory: allocation failed");
   HIPCHK(h, hipGetDevice(&h->dev));
   HIPCHK(h, hipStreamCreate(&h->st));
   {
@@ -1361,7 +1370,7 @@ int lh_create(const lh_config* c, lh_handle** out) {
   // the column-stage jobs of the three substeps (every buffer they name exists now)
   {
     std::vector<ColJob> jobs;
-    for (int k = 0; k < 3; ++k) jobs.push_back(make_job(h, k, 0));
+    for (int k = 0; k < 3; ++k) jobs.push_back(make_job(h, k, 0, h->hio));
     const std::vector<int> map(col_blocks(h), 0);
     HIPCHK(h, attr_col(h));
     HIPCHK(h, hipMalloc((void**)&h->coljobs, jobs.size() * sizeof(ColJob)));
@@ -1405,7 +1414,7 @@ int lh_destroy(lh_handle* h) {
   if (h->twx64) hipFree(h->twx64);
   if (h->twz64) hipFree(h->twz64);
   if (h->st) hipStreamDestroy(h->st);
-  if (h->staged) host_stage().release();
+  if (h->hio) host_stage().release(h->hio);
   delete h;
   return LH_OK;
 }
@@ -1506,14 +1515,12 @@ int lh_substep(lh_handle* h, int krk, double dt) {
   // meanflow_ctP follows the last substep of a step (littleharsh.f90:193-197)
   if (krk == 3 && h->flag_ctpress == 1)
     hipLaunchKernelGGL(k_flowrate, dim3(1), dim3(256), 0, h->st, (const ColJob*)h->coljobs);
+  if (krk == 1) hipLaunchKernelGGL(k_scalars_out, dim3(1), dim3(64), 0, h->st, (const double*)h->scal, h->hio);
   HIPCHK(h, hipGetLastError());
   HIPCHK(h, hipStreamSynchronize(h->st));
   tflush(h);
-  if (krk == 1) {   // the first substep takes the CFL maximum of the state
-    double s[S_NSCAL];
-    return numeric_check(h, false, s);
-  }
-  return LH_OK;
+  // the first substep takes the CFL maximum of the state
+  return krk == 1 ? check_scalars(h, false, h->hio) : LH_OK;
 }
 
 static int run_graph(lh_handle* h, int mode) {
@@ -1538,28 +1545,26 @@ static int run_graph(lh_handle* h, int mode) {
 int lh_step(lh_handle* h, double dt) {
   if (!h) return LH_ERR_ARG;
   if (!(dt > 0.0)) return fail(h, LH_ERR_ARG, "dt must be positive");
-  hipLaunchKernelGGL(k_set_scalar, dim3(1), dim3(1), 0, h->st, h->scal, (int)S_DT, dt);
+  h->hio[kHioIn] = dt;                     // (no earlier step is in flight: every call waits for its own)
   int r = run_graph(h, 0);
   if (r) return r;
   HIPCHK(h, hipGetLastError());
   HIPCHK(h, hipStreamSynchronize(h->st));
   tflush(h);
-  double s[S_NSCAL];
-  return numeric_check(h, false, s);
+  return check_scalars(h, false, h->hio);
 }
 
 int lh_step_cfl(lh_handle* h, double cfl, double* dt_used) {
   if (!h) return LH_ERR_ARG;
   if (!(cfl > 0.0)) return fail(h, LH_ERR_ARG, "cfl must be positive");
-  hipLaunchKernelGGL(k_set_scalar, dim3(1), dim3(1), 0, h->st, h->scal, (int)S_CFL, cfl);
+  h->hio[kHioIn] = cfl;
   int r = run_graph(h, 1);
   if (r) return r;
   HIPCHK(h, hipGetLastError());
   HIPCHK(h, hipStreamSynchronize(h->st));
   tflush(h);
-  double s[S_NSCAL];
-  r = numeric_check(h, true, s);
-  if (dt_used) *dt_used = s[S_DT];
+  r = check_scalars(h, true, h->hio);
+  if (dt_used) *dt_used = h->hio[S_DT];
   return r;
 }
 
@@ -1771,7 +1776,7 @@ int lh_autotune(lh_handle* h, int steps) {
   hipEvent_t e0, e1;
   HIPCHK(h, hipEventCreate(&e0));
   HIPCHK(h, hipEventCreate(&e1));
-  hipLaunchKernelGGL(k_set_scalar, dim3(1), dim3(1), 0, h->st, h->scal, (int)S_CFL, 0.5);
+  h->hio[kHioIn] = 0.5;
   auto trial = [&](float* ms) -> int {
     issue_step(h, true);
     HIPCHK(h, hipEventRecord(e0, h->st));
@@ -1849,7 +1854,7 @@ struct lh_batch {
   int* colmap = nullptr;        // block -> member of the column launches
   int nblk = 0;
   IbSets ib;                    // canopy-stage job tables of the members with small grids
-  double* dscal = nullptr;      // [n][S_NSCAL] the members' scalars after a step
+  double* hscal = nullptr;      // [n][S_NSCAL] the members' scalars after a step (pinned)
   bool joined = false;          // the handles count this batch (in_batch)
   std::string err;
 };
@@ -1909,7 +1914,7 @@ int lh_batch_step_cfl(lh_batch* b, double cfl) {
       for (int i = 0; i < n; ++i) {
         lh_handle* h = b->hs[i];
         if (col_kind(h) != kind) continue;
-        for (int k = 0; k < 3; ++k) jobs[(size_t)k * n + i] = make_job(h, k, nblk);
+        for (int k = 0; k < 3; ++k) jobs[(size_t)k * n + i] = make_job(h, k, nblk, nullptr);
         const int nb = col_blocks(h);
         colmap.insert(colmap.end(), nb, i);
         nblk += nb;
@@ -1928,7 +1933,7 @@ int lh_batch_step_cfl(lh_batch* b, double cfl) {
       return LH_ERR_HIP;
     b->nblk = nblk;
     if (!chk(b->ib.build(b->hs), "canopy job tables")) return LH_ERR_HIP;
-    if (!b->dscal && !chk(hipMalloc((void**)&b->dscal, (size_t)n * S_NSCAL * sizeof(double)), "scalars"))
+    if (!b->hscal && !chk(hipHostMalloc((void**)&b->hscal, (size_t)n * S_NSCAL * sizeof(double), hipHostMallocMapped), "scalars"))
       return LH_ERR_HIP;
     // Per substep: each member's nonlinear stage on its own stream (parallel branches), with
     // the canopy stage of the members with large grids; joined on the master stream, the
@@ -1972,7 +1977,7 @@ int lh_batch_step_cfl(lh_batch* b, double cfl) {
         launch_col(g.kind, b->master, jk, (const int*)b->colmap, g.boff, g.nb, g.nc, g.nyu, kColAll);
     }
     hipLaunchKernelGGL(k_flowrate, dim3(n), dim3(256), 0, b->master, (const ColJob*)b->jobs);
-    hipLaunchKernelGGL(k_jobs_scalars, dim3(sb), dim3(64), 0, b->master, (const ColJob*)b->jobs, n, b->dscal);
+    hipLaunchKernelGGL(k_jobs_scalars, dim3(sb), dim3(64), 0, b->master, (const ColJob*)b->jobs, n, b->hscal);
     const bool ended = chk(hipStreamEndCapture(b->master, &g), "end capture");
     if (!ok || !ended) return LH_ERR_HIP;
     if (!chk(hipGraphInstantiate(&b->g, g, nullptr, nullptr, 0), "instantiate")) {
@@ -1988,14 +1993,8 @@ int lh_batch_step_cfl(lh_batch* b, double cfl) {
     b->err = "batch graph launch failed";
     return LH_ERR_HIP;
   }
-  // every member's scalars in one copy
-  std::vector<double> sc(b->hs.size() * S_NSCAL);
-  if (hipMemcpy(sc.data(), b->dscal, sc.size() * sizeof(double), hipMemcpyDeviceToHost) != hipSuccess) {
-    b->err = "batch scalars: copy failed";
-    return LH_ERR_HIP;
-  }
   for (size_t i = 0; i < b->hs.size(); ++i) {
-    const int r = check_scalars(b->hs[i], true, sc.data() + i * S_NSCAL);
+    const int r = check_scalars(b->hs[i], true, b->hscal + i * S_NSCAL);
     if (r != LH_OK) {
       b->err = "instance " + std::to_string(i) + ": " + b->hs[i]->err;
       return r;
@@ -2014,7 +2013,7 @@ int lh_batch_destroy(lh_batch* b) {
   if (b->g) (void)hipGraphExecDestroy(b->g);
   if (b->jobs) (void)hipFree(b->jobs);
   if (b->colmap) (void)hipFree(b->colmap);
-  if (b->dscal) (void)hipFree(b->dscal);
+  if (b->hscal) (void)hipHostFree(b->hscal);
   b->ib.release();
   for (auto e : b->ev)
     if (e) (void)hipEventDestroy(e);

@@ -530,15 +530,15 @@ __device__ __forceinline__ double lane_of(double v, int i) {
 // of the tile from the rows' lanes (v_readlane) with the operations in the order of LU_dec, so
 // that a row costs its division chain and no memory latency (289 planes: 92 us with a load
 // per row, one thread).
-__device__ __forceinline__ void prep_body(const PREP& a, int w, int l) {
-  const double beta = a.bre * gp(a.scal)[S_DT];
+__device__ __forceinline__ void prep_body(const PREP& a, int w, int l, double dt) {
+  const double beta = a.bre * dt;
   const int d = w == 2 ? a.ct.d : 0;
   const int nj = w == 0 ? a.nyu : (w == 1 ? a.nyv : a.ct.ny + 1);
   const gptr<const double> dd = gp(w == 1 ? a.dyv2i : a.dyu2i) + 3 * d;
   const double gw0 = w == 1 ? 0.0 : a.gw0, gw1 = w == 1 ? 0.0 : a.gw1;
   const gptr<double> ay = gp(w == 1 ? a.ayv : a.ayu);
   const gptr<double> u11 = gp(a.ct.work), m3 = u11 + (a.ct.ny + 2);
-  const double bdt = -a.ct.dR * gp(a.scal)[S_DT];
+  const double bdt = -a.ct.dR * dt;
   double a3 = 0.0, y = 0.0;                  // scaled upper and eliminated rhs of the row before
   for (int t0 = 0; t0 < nj; t0 += 64) {
     const int r = t0 + l;
@@ -699,6 +699,19 @@ __global__ void __launch_bounds__(256) k_maxdiv(const double2* u1, const double2
 // small scalar kernels (graph-capturable replacements for host writes)
 __global__ void k_set_scalar(double* scal, int idx, double v) {
   if (threadIdx.x == 0) scal[idx] = v;
+}
+// start of a step: the caller's value (the CFL number or the time step, from pinned host memory
+// so that a captured step takes a new one each time) and the cleared CFL maximum
+__global__ void k_step_begin(double* scal, const double* in, int idx) {
+  if (threadIdx.x == 0) {
+    scal[idx] = in[0];
+    scal[S_CFLMAX] = 0.0;
+  }
+}
+// the scalars for the host, into pinned memory: read there after the stream's synchronisation,
+// which a copy of their own would double (25 us)
+__global__ void k_scalars_out(const double* scal, double* out) {
+  if (threadIdx.x < S_NSCAL) out[threadIdx.x] = scal[threadIdx.x];
 }
 __global__ void k_cfl_dt(double* scal) {
   if (threadIdx.x == 0) scal[S_DT] = scal[S_CFL] / scal[S_CFLMAX];

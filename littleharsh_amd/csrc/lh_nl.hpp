@@ -267,6 +267,7 @@ struct ZASM {
   // covers the row-by-row recurrence; as a kernel of its own on a side stream its fork and join
   // cost 15 us a substep
   const PREP* prep;
+  double* cfl;                               // non-null: the time step is still to be formed there
 };
 constexpr int kPrepBlocks = 3;
 
@@ -305,7 +306,11 @@ __global__ void __launch_bounds__((2 * L * Plan<PZ, V>::T))
   if (a.prep) {
     // the first blocks: one system each, on the block's first wave
     if (bid < kPrepBlocks) {
-      if (tid < 64 && (bid < 2 || a.prep->ctu)) prep_body(*a.prep, bid, tid);
+      if (tid >= 64 || (bid == 2 && !a.prep->ctu)) return;
+      const gptr<const double> scal = gp(a.prep->scal);
+      const double dt = a.cfl ? scal[S_CFL] / scal[S_CFLMAX] : scal[S_DT];
+      if (a.cfl && bid == 0 && tid == 0) gp(a.cfl)[S_DT] = dt;   // (nothing else here reads it)
+      prep_body(*a.prep, bid, tid, dt);
       return;
     }
     bid -= kPrepBlocks;
