@@ -4,7 +4,8 @@
 // all work buffers.  lh_substep issues the kernels of one RK3 substep:
 //   NL stage   : k_zinv (u,w,v) -> k_xw576 at 576 points in x, k_xraw2 at the other sizes
 //                (x transforms, six products, CFL max)
-//                -> k_zasm (A/B recombination, forward z transforms -> Nu_new)
+//                -> k_zasm (A/B recombination, forward z transforms -> Nu_new), k_zw576 for FP64
+//                planes of 576 x 576 points
 //   IB stage   : k_rhs_ib (rhs and Lu_y on canopy planes) -> k_zinv -> k_xpass_ib -> k_zfwd
 //   column     : k_prep (LU of the shared velocity matrices) -> k_col (RHS0 + rhs of solveU/V,
 //                the velocity solves, constant-flow-rate correction, solveP, v_corr; two
@@ -28,6 +29,7 @@
 #include "lh_kernels.hpp"
 #include "lh_nl.hpp"
 #include "lh_xw.hpp"
+#include "lh_zw.hpp"
 #include "lh_col.hpp"
 #include "lh_colf.hpp"
 #include "lh_stats.hpp"
@@ -316,6 +318,10 @@ static void launch_xraw_t(lh_handle* h, const XRAW& a, const void* tw) {
 #endif
 template <typename TR> struct XwWaves { static constexpr int value = sizeof(TR) == 8 ? 8 : LH_XW_WAVES32; };
 static bool use_xw(const lh_handle* h) { return h->dm.px == 576; }
+// products in tiles and the one-wave-per-line z assembly: FP64 planes of 576 x 576 points, whose z
+// lines are the waves' 576-point transform (per substep of 384 x 289 x 384, x pass and assembly: 2.09
+// ms, with rows and k_zasm 2.77).  Mixed precision keeps k_zasm's operation order
+static bool use_zw(const lh_handle* h) { return use_xw(h) && h->dm.pz == zw::N && h->prec == LH_PREC_FP64; }
 template <typename TR>
 static void launch_xw_t(lh_handle* h, int want_cfl) {
   XW a{h->zu, h->zw, h->zv, h->zp, sizeof(TR) == 8 ? (const void*)h->twxw : (const void*)h->twxw32,
@@ -325,23 +331,34 @@ static void launch_xw_t(lh_handle* h, int want_cfl) {
   constexpr int W = XwWaves<TR>::value;
   const dim3 grid((unsigned)((waves + W - 1) / W)), block(64 * W);
   const size_t sh = xw_lds_bytes<W, TR>();
-  if (want_cfl)
-    hipLaunchKernelGGL((k_xw576<W, true, TR>), grid, block, sh, h->st, a, h->dm);
-  else
-    hipLaunchKernelGGL((k_xw576<W, false, TR>), grid, block, sh, h->st, a, h->dm);
+  if constexpr (sizeof(TR) == 8) {
+    if (use_zw(h)) {
+      if (want_cfl) hipLaunchKernelGGL((k_xw576<W, true, TR, true>), grid, block, sh, h->st, a, h->dm);
+      else hipLaunchKernelGGL((k_xw576<W, false, TR, true>), grid, block, sh, h->st, a, h->dm);
+      return;
+    }
+  }
+  if (want_cfl) hipLaunchKernelGGL((k_xw576<W, true, TR, false>), grid, block, sh, h->st, a, h->dm);
+  else hipLaunchKernelGGL((k_xw576<W, false, TR, false>), grid, block, sh, h->st, a, h->dm);
 }
 static void launch_xw(lh_handle* h, int want_cfl) {
   if (h->prec == LH_PREC_FP64) launch_xw_t<double>(h, want_cfl);
   else launch_xw_t<float>(h, want_cfl);
 }
-template <typename TR>
+static hipError_t max_lds(const void* kernel, size_t bytes) {
+  return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+}
+template <typename TR, bool TILE>
 static hipError_t attr_xw_t() {
   constexpr int W = XwWaves<TR>::value;
-  hipError_t e = hipFuncSetAttribute((const void*)k_xw576<W, true, TR>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     (int)xw_lds_bytes<W, TR>());
-  if (e != hipSuccess) return e;
-  return hipFuncSetAttribute((const void*)k_xw576<W, false, TR>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                             (int)xw_lds_bytes<W, TR>());
+  const hipError_t e = max_lds((const void*)k_xw576<W, true, TR, TILE>, xw_lds_bytes<W, TR>());
+  return e != hipSuccess ? e : max_lds((const void*)k_xw576<W, false, TR, TILE>, xw_lds_bytes<W, TR>());
+}
+static void launch_zw(lh_handle* h, const ZASM& z) {
+  const Dims& dm = h->dm;
+  ZW a{(const double2*)h->zp, h->twxw, z.nu1, z.nu2, z.nu3, z.dthdyu, z.dthdyv, z.k1x, z.k1z, z.lc, z.prep, z.cfl};
+  const int nb = zw::groups(dm.mx) * ((dm.nyu - 2 + a.lc - 1) / a.lc) + (a.prep ? kPrepBlocks : 0);
+  hipLaunchKernelGGL(k_zw576, dim3(nb), dim3(512), zw::lds_bytes(), h->st, a, dm);
 }
 // the canopy x pass at 576 points: one wave per (entry, row pair), LH_XIBW_WAVES per block
 // (12: three per SIMD at 132 VGPRs, 121 KB of LDS; 16 would spill)
@@ -996,7 +1013,9 @@ static void issue_substep(lh_handle* h, int krk /*0-based*/, bool cfl_mode, int 
     // in: six product Z rows per level; out: Nu_new
     const double by = 6.0 * nlev * zsl + spl * (2.0 * nlev + (nlev - 1));
     TIMED(h, LH_K_ASM, by, {
-      if (f64) {
+      if (use_zw(h)) {
+        launch_zw(h, a);
+      } else if (f64) {
         LH_DISPATCH_PLAN(dm.pz, h->zplan, launch_zasm_t, double, h, a, h->twz)
       } else {
         LH_DISPATCH_PLAN(dm.pz, h->zplan, launch_zasm_t, float, h, a, h->twz)
@@ -1168,7 +1187,9 @@ int lh_create(const lh_config* c, lh_handle** out) {
       // one block of kXwWaves waves per CU; a chunk's start-up is three inverse transforms
       // against nine transforms per level
       const bool f64 = h->prec == LH_PREC_FP64;
-      HIPCHK(h, f64 ? attr_xw_t<double>() : attr_xw_t<float>());
+      const hipError_t ea = !f64 ? attr_xw_t<float, false>() : (use_zw(h) ? attr_xw_t<double, true>() : attr_xw_t<double, false>());
+      HIPCHK(h, ea);
+      if (use_zw(h)) HIPCHK(h, max_lds((const void*)k_zw576, zw::lds_bytes()));
       HIPCHK(h, hipFuncSetAttribute((const void*)k_xpass_ib576<LH_XIBW_WAVES>,
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)xibw_lds_bytes()));
       const int wpb = f64 ? XwWaves<double>::value : XwWaves<float>::value;
@@ -1176,6 +1197,8 @@ int lh_create(const lh_config* c, lh_handle** out) {
         h->xraw_lc = chunk_levels(dm.nyu - 2, (long)dm.pz / 2, ncu * wpb, 4, 96, 1.0 / 3.0);
     }
     if (h->xraw_lc <= 0) h->xraw_lc = chunk_levels(dm.nyu - 2, dm.pz / 2, ncu * bx, 4, 64, 1.0);
+    // the wave assembly: one block per CU; a chunk's start-up is half a level (three tiles of six)
+    if (h->zasm_lc <= 0 && use_zw(h)) h->zasm_lc = chunk_levels(dm.nyu - 2, zw::groups(dm.mx), ncu, 2, 96, 0.5);
     if (h->zasm_lc <= 0)
       h->zasm_lc = chunk_levels(dm.nyu - 2, 3L * ((dm.mx + LH_ZASM_COLS - 1) / LH_ZASM_COLS), ncu * bz, 2, 12, 0.25);
   }
@@ -1222,7 +1245,7 @@ int lh_create(const lh_config* c, lh_handle** out) {
   HIPCHK(h, hipMalloc(&h->zv, zel * zslot * dm.nyv));
   // zp also serves as the FP64 scratch of the IB stage
   {
-    size_t nzp = zel * zslot * 6 * (size_t)nlev;
+    size_t nzp = use_zw(h) ? zel * zw::zp_values(nlev, dm.mx) : zel * zslot * 6 * (size_t)nlev;
     size_t nib = sizeof(double2) * zslot * (3 * (size_t)dm.nyu + 6);
     HIPCHK(h, hipMalloc(&h->zp, nzp > nib ? nzp : nib));
   }

@@ -70,6 +70,13 @@ struct ColF {
     v.y = a.y;
     *reinterpret_cast<D2 __attribute__((address_space(1)))*>(b + o) = v;
   }
+  // (a store of values that nothing reads before they have left the caches)
+  __device__ __forceinline__ void st_nt(unsigned o, double2 a) const {
+    D2 v;
+    v.x = a.x;
+    v.y = a.y;
+    __builtin_nontemporal_store(v, reinterpret_cast<D2 __attribute__((address_space(1)))*>(b + o));
+  }
 };
 
 // PRE: every row a thread reads is loaded ahead of the first barrier (small R: the chain of

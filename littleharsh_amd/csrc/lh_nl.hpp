@@ -15,9 +15,9 @@
 //   w:  A3 = ikx uw + m_u (vw - vw_prev),   B3 = ww
 //   v:  A2 = ikx uv_prev + m_v (vv - vv_prev), B2 = vw_prev   (face j-1 at level j)
 // The x pass (k_xraw2) produces the six raw products per level (their x spectra, two rows
-// packed per complex transform); the forward z pass (k_zasm) separates the rows, forms A
-// and B and transforms them into Nu_new.  RHS0 and the rhs of solveU/solveV are built
-// inside the velocity sweeps (k_vel_rhs, lh_col.hpp).
+// packed per complex transform); the forward z pass (k_zasm; lh_zw.hpp has the one of FP64 planes
+// of 576 x 576 points) separates the rows, forms A and B and transforms them into Nu_new.  RHS0 and
+// the rhs of solveU/solveV are built inside the column stage (lh_colf.hpp, lh_col.hpp).
 #pragma once
 #include <type_traits>
 #include "lh_kernels.hpp"
@@ -270,6 +270,14 @@ struct ZASM {
   double* cfl;                               // non-null: the time step is still to be formed there
 };
 constexpr int kPrepBlocks = 3;
+// the extra blocks: one system each, on the block's first wave; cfl as in ZASM
+__device__ __forceinline__ void prep_block(const PREP& p, double* cfl, int w, int lane) {
+  if (w == 2 && !p.ctu) return;
+  const gptr<const double> scal = gp(p.scal);
+  const double dt = cfl ? scal[S_CFL] / scal[S_CFLMAX] : scal[S_DT];
+  if (cfl && w == 0 && lane == 0) gp(cfl)[S_DT] = dt;     // (nothing else in the launch reads it)
+  prep_body(p, w, lane, dt);
+}
 
 // twiddle table of the z assembly's transforms
 template <int PZ, typename C, int V = 0>
@@ -304,13 +312,8 @@ __global__ void __launch_bounds__((2 * L * Plan<PZ, V>::T))
   const int nlev = dm.nyu - 2;
   int bid = blockIdx.x;
   if (a.prep) {
-    // the first blocks: one system each, on the block's first wave
     if (bid < kPrepBlocks) {
-      if (tid >= 64 || (bid == 2 && !a.prep->ctu)) return;
-      const gptr<const double> scal = gp(a.prep->scal);
-      const double dt = a.cfl ? scal[S_CFL] / scal[S_CFLMAX] : scal[S_DT];
-      if (a.cfl && bid == 0 && tid == 0) gp(a.cfl)[S_DT] = dt;   // (nothing else here reads it)
-      prep_body(*a.prep, bid, tid, dt);
+      if (tid < 64) prep_block(*a.prep, a.cfl, bid, tid);
       return;
     }
     bid -= kPrepBlocks;

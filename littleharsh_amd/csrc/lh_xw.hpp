@@ -25,6 +25,7 @@
 // A wave's LDS operations complete in issue order, so the transposes need no barrier; the
 // empty asm statements only keep the compiler from moving memory accesses across them.
 #pragma once
+#include "lh_colf.hpp"
 #include "lh_kernels.hpp"
 
 namespace lh {
@@ -277,9 +278,11 @@ template <typename C> __device__ __forceinline__ void fwd576(C (&v)[9], int t, C
 // Every lane issues every load (no load is left to one lane), so that the line waits for
 // memory once: lane 0's mode 0 drops the imaginary parts, and mode 192 (lane 0 of slot 3;
 // the other lanes of that slot are zero padding), by factors 0 and 1.
-template <typename C> __device__ __forceinline__ void load_line(C (&v)[9], const C* __restrict__ A, int t) {
+// (the second row `second` values after the first)
+template <typename C>
+__device__ __forceinline__ void load_line(C (&v)[9], const C* __restrict__ A, int t, size_t second = MX) {
   using R = decltype(C::x);
-  const C* B = A + MX;
+  const C* B = A + second;
   const R lane0 = t == 0 ? (R)1 : (R)0, other = (R)1 - lane0;
   C a[3], b[3];
 #pragma unroll
@@ -310,6 +313,24 @@ template <typename C> __device__ __forceinline__ void store_line(const C (&v)[9]
   if (t == 0) dst[192] = v[3];
 #pragma unroll
   for (int r = 6; r < 9; ++r) dst[MX + N - (t + 64 * r)] = v[r];
+}
+
+// the same as one row pair of the product tiles of lh_zw.hpp (dst: the pair's place in the tile of
+// group 0): column k in group k / 8, GROUP values apart, at k % 8 of its sixteen values, P[576 - k]
+// eight further.  GROUP holds one row pair more than the plane has, so that the groups of one store
+// start on different L2 channels; the stores leave no lines in the caches, which the 3.2 GB of a
+// substep would only sweep (the launch at 384 x 289 x 384: 1.21 ms without either, 1.19 with the
+// stride, 1.12 with both; whole rows 1.11)
+constexpr int GROUP = 289 * 16;
+__device__ __forceinline__ void store_tile(const double2 (&v)[9], const double2* dst, int t) {
+  const unsigned oa = (unsigned)((t >> 3) * GROUP + (t & 7)) * 16u;
+  const int k = 192 - t;
+  const unsigned ob = (unsigned)((k >> 3) * GROUP + (k & 7)) * 16u;
+#pragma unroll
+  for (int r = 0; r < 3; ++r) ColF(dst + 8 * r * GROUP).st_nt(oa, v[r]);
+  if (t == 0) ColF(dst + 24 * GROUP).st(0u, v[3]);
+#pragma unroll
+  for (int r = 6; r < 9; ++r) ColF(dst + 8 + 8 * (6 - r) * GROUP).st_nt(ob, v[r]);
 }
 
 }  // namespace xw
@@ -343,7 +364,9 @@ template <typename TR, int WPB> constexpr int xw_wpe() { return sizeof(TR) == 8 
 // by slot as an operand.
 // CFL: whether the launch forms the CFL maximum (a template flag, so that the slot loops
 // carry no branch on it)
-template <int WPB, bool CFL, typename TR>
+// TILE: rows z and z + pz / 2 pair up and the products go out in the tiles of lh_zw.hpp (otherwise
+// rows 2 z and 2 z + 1, and whole rows)
+template <int WPB, bool CFL, typename TR, bool TILE>
 __global__ void __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(xw_wpe<TR, WPB>())))
     k_xw576(XW a, Dims dm) {
   using C = cx<TR>;
@@ -358,14 +381,14 @@ __global__ void __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(x
   C* buf = lds + xw::TWN + wv * (xw::LINE + 9 * 64);
   C* pk = buf + xw::LINE + t;                    // park line: slot s at pk[64 s]
   const int nlev = dm.nyu - 2;
-  const int npair = dm.pz / 2;
+  const int npair = TILE ? 288 : dm.pz / 2;          // tiles: planes of 576 rows
   const int item = blockIdx.x * WPB + wv;
   const int pair = item % npair, chunk = item / npair;
   const int l0 = chunk * a.lc;
   const int l1 = min(l0 + a.lc, nlev);
   if (l0 >= l1) return;
-  const size_t slot = (size_t)dm.pz * xw::MX;
-  const size_t row = (size_t)pair * 2 * xw::MX;
+  const size_t slot = (size_t)(2 * npair) * xw::MX;
+  const size_t row = (size_t)pair * (TILE ? 1 : 2) * xw::MX, second = TILE ? (size_t)npair * xw::MX : (size_t)xw::MX;
   const C* zu = static_cast<const C*>(a.zu);
   const C* zw = static_cast<const C*>(a.zw);
   const C* zv = static_cast<const C*>(a.zv);
@@ -381,19 +404,23 @@ __global__ void __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(x
   };
   auto out = [&](int q, int l, C (&x)[9]) {
     xw::fwd576(x, t, buf, tw);
-    xw::store_line(x, zp + ((size_t)q * nlev + l) * slot + row, t);
+    if constexpr (TILE) {
+      xw::store_tile(x, zp + ((size_t)q * nlev + l) * ((xw::MX + 7) / 8) * xw::GROUP + pair * 16, t);
+    } else {
+      xw::store_line(x, zp + ((size_t)q * nlev + l) * slot + row, t);
+    }
   };
-  xw::load_line(cu, zu + (size_t)(l0 + 1) * slot + row, t);
+  xw::load_line(cu, zu + (size_t)(l0 + 1) * slot + row, t, second);
   xw::inv576(cu, t, buf, tw);
-  xw::load_line(cw, zw + (size_t)(l0 + 1) * slot + row, t);
+  xw::load_line(cw, zw + (size_t)(l0 + 1) * slot + row, t, second);
   xw::inv576(cw, t, buf, tw);
-  xw::load_line(p, zv + (size_t)l0 * slot + row, t);
+  xw::load_line(p, zv + (size_t)l0 * slot + row, t, second);
   xw::inv576(p, t, buf, tw);
   park(p);                                        // V(j-1)
   for (int l = l0; l < l1; ++l) {
     // V(j), the face above: vv and the CFL maximum at the centre, from V(j-1) parked
     C vj[9];
-    xw::load_line(vj, zv + (size_t)(l + 1) * slot + row, t);
+    xw::load_line(vj, zv + (size_t)(l + 1) * slot + row, t, second);
     xw::inv576(vj, t, buf, tw);
 #pragma unroll
     for (int s = 0; s < 9; ++s) {
@@ -435,7 +462,7 @@ __global__ void __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(x
     }
     out(2, l, p);
     // U(j+1): uv at the face, then carried
-    xw::load_line(p, zu + (size_t)(l + 2) * slot + row, t);
+    xw::load_line(p, zu + (size_t)(l + 2) * slot + row, t, second);
     xw::inv576(p, t, buf, tw);
 #pragma unroll
     for (int s = 0; s < 9; ++s) {
@@ -447,7 +474,7 @@ __global__ void __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(x
     for (int s = 0; s < 9; ++s) cu[s] = p[s];
     // W(j+1): vw at the face, then carried; W(j) comes back from the park line, which then
     // takes V(j) for the next level
-    xw::load_line(p, zw + (size_t)(l + 2) * slot + row, t);
+    xw::load_line(p, zw + (size_t)(l + 2) * slot + row, t, second);
     xw::inv576(p, t, buf, tw);
     xw::mem_fence_compiler();
 #pragma unroll
