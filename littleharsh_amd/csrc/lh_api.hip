@@ -29,6 +29,7 @@
 #include "lh_kernels.hpp"
 #include "lh_nl.hpp"
 #include "lh_xw.hpp"
+#include "lh_xs.hpp"
 #include "lh_zw.hpp"
 #include "lh_col.hpp"
 #include "lh_colf.hpp"
@@ -135,6 +136,7 @@ struct lh_handle {
   hipGraphExec_t gexec[2] = {nullptr, nullptr};   // [0] fixed dt, [1] device CFL dt
   double graph_dt = -1.0;
   // launch parameters (lh_autotune picks them per instance)
+  int ncu = 1;                                  // compute units
   int xraw_lc = LH_XRAW_LC;
   int zasm_lc = LH_ZASM_LC;
   int col_bs = LH_COL_BS;
@@ -345,6 +347,34 @@ static void launch_xw(lh_handle* h, int want_cfl) {
   if (h->prec == LH_PREC_FP64) launch_xw_t<double>(h, want_cfl);
   else launch_xw_t<float>(h, want_cfl);
 }
+// the same in FP64 at the other lengths: F::LPW row pairs per wave.  With one level per wave the
+// products are shared out over three waves where all of them are resident at once, two per SIMD (per
+// launch of 32 x 41 x 32 with 351 of them: 9.9 us, unsplit 14.1; 48 x 97 x 48, 1710: 17.5, 20.5;
+// 64 x 97 x 64, 2850: 23.6 either way; 96 x 145 x 96, 6435: 49.6, two levels per wave unsplit 48)
+#define LH_DISPATCH_XS(n, F, ...)          \
+  switch (n) {                             \
+    case 48: F<48>(__VA_ARGS__); break;    \
+    case 72: F<72>(__VA_ARGS__); break;    \
+    case 96: F<96>(__VA_ARGS__); break;    \
+    case 144: F<144>(__VA_ARGS__); break;  \
+    case 384: F<384>(__VA_ARGS__); break;  \
+    default: break;                        \
+  }
+template <int N> static void launch_xs_t(lh_handle* h, int want_cfl) {
+  using F = xs::Family<N>;
+  XW a{h->zu, h->zw, h->zv, h->zp, h->twx, h->dthdyu, h->scal, want_cfl, h->xraw_lc};
+  const long groups = (h->dm.pz / 2 + F::LPW - 1) / F::LPW, nlev = h->dm.nyu - 2;
+  if (a.lc == 1 && xs::kSplitWaves * groups * nlev <= 8L * h->ncu) {
+    const dim3 grid((unsigned)(groups * nlev)), block(64 * xs::kSplitWaves);
+    if (want_cfl) hipLaunchKernelGGL((k_xs_split<N, true>), grid, block, xs::split_lds_bytes<F>(), h->st, a, h->dm);
+    else hipLaunchKernelGGL((k_xs_split<N, false>), grid, block, xs::split_lds_bytes<F>(), h->st, a, h->dm);
+    return;
+  }
+  const long waves = groups * ((nlev + a.lc - 1) / a.lc);
+  const dim3 grid((unsigned)((waves + F::WPB - 1) / F::WPB)), block(64 * F::WPB);
+  if (want_cfl) hipLaunchKernelGGL((k_xs<N, true>), grid, block, xs::lds_bytes<F>(), h->st, a, h->dm);
+  else hipLaunchKernelGGL((k_xs<N, false>), grid, block, xs::lds_bytes<F>(), h->st, a, h->dm);
+}
 static hipError_t max_lds(const void* kernel, size_t bytes) {
   return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
 }
@@ -353,6 +383,19 @@ static hipError_t attr_xw_t() {
   constexpr int W = XwWaves<TR>::value;
   const hipError_t e = max_lds((const void*)k_xw576<W, true, TR, TILE>, xw_lds_bytes<W, TR>());
   return e != hipSuccess ? e : max_lds((const void*)k_xw576<W, false, TR, TILE>, xw_lds_bytes<W, TR>());
+}
+template <int N> static void attr_xs_t(hipError_t* e) {
+  constexpr size_t sh = xs::lds_bytes<xs::Family<N>>();
+  *e = max_lds((const void*)k_xs<N, true>, sh);
+  if (*e == hipSuccess) *e = max_lds((const void*)k_xs<N, false>, sh);
+  constexpr size_t sp = xs::split_lds_bytes<xs::Family<N>>();
+  static_assert(sp <= 64 * 1024, "within the default limit");
+}
+// levels per wave: F::CAP waves per CU; a chunk's start-up is three inverse transforms against nine
+// transforms per level
+template <int N> static void xs_levels_t(lh_handle* h, int ncu) {
+  using F = xs::Family<N>;
+  h->xraw_lc = chunk_levels(h->dm.nyu - 2, (h->dm.pz / 2 + F::LPW - 1) / F::LPW, ncu * F::CAP, 1, 96, 1.0 / 3.0);
 }
 static void launch_zw(lh_handle* h, const ZASM& z) {
   const Dims& dm = h->dm;
@@ -482,6 +525,19 @@ static void launch_zfwd(lh_handle* h, const ZJobs& jobs, int njobs, int maxn, bo
     LH_DISPATCH_PLAN(h->dm.pz, h->zplan, launch_zfwd_t, double, h, jobs, njobs, maxn, fp64 ? h->twz64 : h->twz)
   } else {
     LH_DISPATCH_PLAN(h->dm.pz, h->zplan, launch_zfwd_t, float, h, jobs, njobs, maxn, h->twz)
+  }
+}
+
+// x pass of the nonlinear stage
+static void launch_x(lh_handle* h, int want_cfl) {
+  const Dims& dm = h->dm;
+  if (use_xw(h)) {
+    launch_xw(h, want_cfl);
+  } else if (h->prec == LH_PREC_FP64) {
+    LH_DISPATCH_XS(dm.px, launch_xs_t, h, want_cfl)
+  } else {
+    XRAW a{h->zu, h->zw, h->zv, h->zp, h->dthdyu, h->scal, want_cfl};
+    LH_DISPATCH_PLAN(dm.px, h->xplan, launch_xraw_t, float, h, a, h->twx)
   }
 }
 
@@ -984,18 +1040,7 @@ static void issue_substep(lh_handle* h, int krk /*0-based*/, bool cfl_mode, int 
   if (krk == 0 && !(stages & (kCallerCfl | kBegun)))
     TIMED(h, LH_K_MISC, 0.0,
           hipLaunchKernelGGL(k_set_scalar, dim3(1), dim3(1), 0, h->st, h->scal, (int)S_CFLMAX, 0.0));
-  {
-    XRAW a{h->zu, h->zw, h->zv, h->zp, h->dthdyu, h->scal, krk == 0 ? 1 : 0};
-    TIMED(h, LH_K_XNL, nuvw * zsl + 6.0 * nlev * zsl, {
-      if (use_xw(h)) {
-        launch_xw(h, krk == 0 ? 1 : 0);
-      } else if (f64) {
-        LH_DISPATCH_PLAN(dm.px, h->xplan, launch_xraw_t, double, h, a, h->twx)
-      } else {
-        LH_DISPATCH_PLAN(dm.px, h->xplan, launch_xraw_t, float, h, a, h->twx)
-      }
-    });
-  }
+  TIMED(h, LH_K_XNL, nuvw * zsl + 6.0 * nlev * zsl, launch_x(h, krk == 0 ? 1 : 0));
   if (krk == 0 && cfl_mode && !(stages & kCallerCfl) && !prep_in_asm(stages))
     TIMED(h, LH_K_MISC, 0.0, hipLaunchKernelGGL(k_cfl_dt, dim3(1), dim3(1), 0, h->st, h->scal));
   }
@@ -1164,12 +1209,11 @@ int lh_create(const lh_config* c, lh_handle** out) {
       LH_DISPATCH_PLAN(c->pz, v, attr_z_t, float, &dummy)
     }
     for (int v = 0; v < plans_of_len(c->px); ++v) {
-      LH_DISPATCH_PLAN(c->px, v, attr_xraw_t, double, &dummy)
       LH_DISPATCH_PLAN(c->px, v, attr_xraw_t, float, &dummy)
     }
   }
   {
-    int ncu = 0;
+    int& ncu = h->ncu;
     HIPCHK(h, hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, h->dev));
     if (ncu < 1) ncu = 1;
     // slots = CUs x resident blocks per CU of the kernel at its precision
@@ -1178,7 +1222,6 @@ int lh_create(const lh_config* c, lh_handle** out) {
       LH_DISPATCH_PLAN(dm.px, h->xplan, xraw_occ_t, float, &bx)
       LH_DISPATCH_PLAN(dm.pz, h->zplan, zasm_occ_t, float, &bz)
     } else {
-      LH_DISPATCH_PLAN(dm.px, h->xplan, xraw_occ_t, double, &bx)
       LH_DISPATCH_PLAN(dm.pz, h->zplan, zasm_occ_t, double, &bz)
     }
     if (bx < 1) bx = 1;
@@ -1195,6 +1238,12 @@ int lh_create(const lh_config* c, lh_handle** out) {
       const int wpb = f64 ? XwWaves<double>::value : XwWaves<float>::value;
       if (h->xraw_lc <= 0)
         h->xraw_lc = chunk_levels(dm.nyu - 2, (long)dm.pz / 2, ncu * wpb, 4, 96, 1.0 / 3.0);
+    }
+    if (!use_xw(h) && h->prec == LH_PREC_FP64) {
+      hipError_t ex = hipSuccess;
+      LH_DISPATCH_XS(dm.px, attr_xs_t, &ex)
+      HIPCHK(h, ex);
+      if (h->xraw_lc <= 0) LH_DISPATCH_XS(dm.px, xs_levels_t, h, ncu)
     }
     if (h->xraw_lc <= 0) h->xraw_lc = chunk_levels(dm.nyu - 2, dm.pz / 2, ncu * bx, 4, 64, 1.0);
     // the wave assembly: one block per CU; a chunk's start-up is half a level (three tiles of six)
@@ -1625,14 +1674,7 @@ int lh_cfl_dt(lh_handle* h, double cfl, double* dt) {
   jobs.j[1] = ZJob{h->u3, h->zw, nullptr, 0, dm.nyu, 0};
   jobs.j[2] = ZJob{h->u2, h->zv, nullptr, 0, dm.nyv, 0};
   launch_zinv(h, jobs, 3, dm.nyu, false);
-  XRAW a{h->zu, h->zw, h->zv, h->zp, h->dthdyu, h->scal, 1};
-  if (use_xw(h)) {
-    launch_xw(h, 1);
-  } else if (h->prec == LH_PREC_FP64) {
-    LH_DISPATCH_PLAN(dm.px, h->xplan, launch_xraw_t, double, h, a, h->twx)
-  } else {
-    LH_DISPATCH_PLAN(dm.px, h->xplan, launch_xraw_t, float, h, a, h->twx)
-  }
+  launch_x(h, 1);
   hipLaunchKernelGGL(k_cfl_dt, dim3(1), dim3(1), 0, h->st, h->scal);
   HIPCHK(h, hipGetLastError());
   HIPCHK(h, hipStreamSynchronize(h->st));
