@@ -2,11 +2,13 @@
 //
 // The handle owns one HIP stream, the device-resident state in [plane][column] layout and
 // all work buffers.  lh_substep issues the kernels of one RK3 substep:
-//   NL stage   : k_zinv (u,w,v) -> k_xw576 at 576 points in x, k_xraw2 at the other sizes
+//   NL stage   : k_zinv (u,w,v) -> k_xw576 at 576 points in x, k_xs (k_xraw2 in mixed
+//                precision) at the other sizes
 //                (x transforms, six products, CFL max)
 //                -> k_zasm (A/B recombination, forward z transforms -> Nu_new), k_zw576 for FP64
 //                planes of 576 x 576 points
-//   IB stage   : k_rhs_ib (rhs and Lu_y on canopy planes) -> k_zinv -> k_xpass_ib -> k_zfwd
+//   IB stage   : k_rhs_ib (rhs and Lu_y on canopy planes), then k_ib_plane (FP64, lengths up to
+//                144) or k_zinv -> k_xpass_ib -> k_zfwd
 //   column     : k_prep (LU of the shared velocity matrices) -> k_col (RHS0 + rhs of solveU/V,
 //                the velocity solves, constant-flow-rate correction, solveP, v_corr; two
 //                one-thread-per-column kernels in mixed precision and for very tall channels); these
@@ -30,6 +32,7 @@
 #include "lh_nl.hpp"
 #include "lh_xw.hpp"
 #include "lh_xs.hpp"
+#include "lh_ibp.hpp"
 #include "lh_zw.hpp"
 #include "lh_col.hpp"
 #include "lh_colf.hpp"
@@ -124,6 +127,7 @@ struct lh_handle {
   int nibu = 0, nibv = 0;
   IBEntry* ibent = nullptr;
   int nibent = 0;
+  std::vector<IBEntry> h_ent;     // the entries on the host
   int nibtip = 0;                 // entries with a Lu_y slot (tip planes), stored first
   // statistics and spectra (allocated on first use)
   double *st_psum = nullptr, *st_pfold = nullptr, *st_acc = nullptr, *cst_acc = nullptr;
@@ -830,6 +834,33 @@ static hipError_t attr_col(const lh_handle* h) {
 // batch the channels that share the kernel, the length and the plan form one launch.
 static bool small_channel(const lh_handle* h) { return h->dm.px <= 144 && h->dm.pz <= 144; }
 static bool ib_jobs(const lh_handle* h) { return small_channel(h) && h->nibent > 0; }
+// The planes of such a channel in FP64 run whole, one block each.  (Mixed precision keeps the three
+// kernels and their order of operations: its results follow every rounding of the canopy rhs.)
+static bool ib_plane(const lh_handle* h) { return ib_jobs(h) && h->prec == LH_PREC_FP64; }
+#define LH_IBP_ROW(px, pz, F, ...)             \
+  switch (pz) {                                \
+    case 48: F<px, 48>(__VA_ARGS__); break;    \
+    case 72: F<px, 72>(__VA_ARGS__); break;    \
+    case 96: F<px, 96>(__VA_ARGS__); break;    \
+    case 144: F<px, 144>(__VA_ARGS__); break;  \
+    default: break;                            \
+  }
+#define LH_DISPATCH_IBP(px, pz, F, ...)               \
+  switch (px) {                                       \
+    case 48: LH_IBP_ROW(48, pz, F, __VA_ARGS__) break;    \
+    case 72: LH_IBP_ROW(72, pz, F, __VA_ARGS__) break;    \
+    case 96: LH_IBP_ROW(96, pz, F, __VA_ARGS__) break;    \
+    case 144: LH_IBP_ROW(144, pz, F, __VA_ARGS__) break;  \
+    default: break;                                   \
+  }
+template <int PX, int PZ> static void launch_ibp_t(hipStream_t st, const IbpJob* jt, int nblk) {
+  using S = ibp::Shape<PX, PZ>;
+  hipLaunchKernelGGL((k_ib_plane<PX, PZ>), dim3(nblk), dim3(64 * S::WAVES), S::LDS, st, jt);
+}
+template <int PX, int PZ> static void attr_ibp_t(hipError_t* e) {
+  static_assert(ibp::Shape<PX, PZ>::LDS <= 160 * 1024, "a plane fits the LDS");
+  *e = max_lds((const void*)k_ib_plane<PX, PZ>, ibp::Shape<PX, PZ>::LDS);
+}
 template <int N, typename TR, int V> static void zlines_of_t(int* l) { *l = zlines<N, V>(); }
 static int zlines_of(int n, int v) {
   int l = 16;
@@ -940,10 +971,22 @@ static XIB ib_xib(const lh_handle* h, int krk, int paired) {
 }
 static int zgrid_cols(const lh_handle* h) { return (h->dm.mx + zlines_of(h->dm.pz, h->zplan) - 1) / zlines_of(h->dm.pz, h->zplan); }
 
+static int ibp_units(const lh_handle* h) { return ib_plane(h) ? h->nibent : 0; }
+static IbpJob ibp_job(const lh_handle* h, int u, int krk) {
+  const IBEntry& en = h->h_ent[u];
+  const int f = en.slot < h->nibu ? 0 : (en.slot < 2 * h->nibu ? 1 : 2);
+  const int plane = f == 2 ? h->h_ibv[en.slot - 2 * h->nibu] : h->h_ibu[en.slot - f * h->nibu];
+  const size_t ncol = h->dm.ncol;
+  return IbpJob{(f == 0 ? h->r1 : (f == 1 ? h->r3 : h->r2)) + plane * ncol,
+                en.lslot < 0 ? nullptr : h->tipl + (en.lslot - 2 * h->nibu - h->nibv) * ncol,
+                h->masks + (size_t)en.mask * h->dm.pz * h->dm.px, h->scal, (const double2*)h->twx64,
+                (const double2*)h->twz64, h->rk[3 + krk] / h->dm.re};
+}
 struct IbSets {
   GroupSet<RhsIbJob> ri;
   GroupSet<ZJobT> zi, zf;
   GroupSet<XibJob> xb;
+  GroupSet<IbpJob> pl;
   hipError_t build(const std::vector<lh_handle*>& hs) {
     hipError_t e = ri.build(
         hs, 1, 3, [](const lh_handle* h, int, int* l, int* v) { *l = 0; *v = 0; return ib_jobs(h); },
@@ -953,14 +996,14 @@ struct IbSets {
         });
     if (e == hipSuccess)
       e = zi.build(
-          hs, 1, 1, [](const lh_handle* h, int, int* l, int* v) { *l = h->dm.pz; *v = h->zplan; return ib_jobs(h); },
+          hs, 1, 1, [](const lh_handle* h, int, int* l, int* v) { *l = h->dm.pz; *v = h->zplan; return ib_jobs(h) && !ib_plane(h); },
           [](const lh_handle* h, int) { return zgrid_cols(h) * ib_maxn(h) * 4; },
           [](const lh_handle* h, int, int, int blk0) {
             return ZJobT{ib_zinv_jobs(h), h->dm, h->twz64, blk0, zgrid_cols(h) * ib_maxn(h) * 4};
           });
     if (e == hipSuccess)
       e = zf.build(
-          hs, 1, 1, [](const lh_handle* h, int, int* l, int* v) { *l = h->dm.pz; *v = h->zplan; return ib_jobs(h); },
+          hs, 1, 1, [](const lh_handle* h, int, int* l, int* v) { *l = h->dm.pz; *v = h->zplan; return ib_jobs(h) && !ib_plane(h); },
           [](const lh_handle* h, int) { return zgrid_cols(h) * ib_npl(h) * 3; },
           [](const lh_handle* h, int, int, int blk0) {
             return ZJobT{ib_zfwd_jobs(h), h->dm, h->twz64, blk0, zgrid_cols(h) * ib_npl(h) * 3};
@@ -972,7 +1015,7 @@ struct IbSets {
           hs, 2, 3,
           [](const lh_handle* h, int u, int* l, int* v) {
             *l = h->dm.px; *v = h->xplan;
-            return ib_jobs(h) && (u == 0 ? h->nibtip > 0 : h->nibent > h->nibtip);
+            return ib_jobs(h) && !ib_plane(h) && (u == 0 ? h->nibtip > 0 : h->nibent > h->nibtip);
           },
           [](const lh_handle* h, int u) {
             return u == 0 ? (h->dm.pz / 2) * h->nibtip : (h->dm.pz / 4) * (h->nibent - h->nibtip);
@@ -980,11 +1023,19 @@ struct IbSets {
           [](const lh_handle* h, int u, int k, int blk0) {
             return XibJob{ib_xib(h, k, u), h->dm, h->twx64, blk0, h->dm.pz / (u == 0 ? 2 : 4)};
           });
+    // whole planes: a unit per block, the tips first
+    int nu = 0;
+    for (const lh_handle* h : hs) nu = std::max(nu, ibp_units(h));
+    if (e == hipSuccess)
+      e = pl.build(
+          hs, nu, 3,
+          [](const lh_handle* h, int u, int* l, int* v) { *l = h->dm.px; *v = h->dm.pz; return u < ibp_units(h); },
+          [](const lh_handle*, int) { return 1; }, [](const lh_handle* h, int u, int k, int) { return ibp_job(h, u, k); });
     return e;
   }
-  void release() { ri.release(); zi.release(); zf.release(); xb.release(); }
+  void release() { ri.release(); zi.release(); zf.release(); xb.release(); pl.release(); }
   // the launches of the canopy stage of substep k of every channel in the sets, in stage
-  // order: rhs, inverse z, x (tip and other entries together), forward z
+  // order: rhs, then whole planes, or inverse z, x (tip and other entries together) and forward z
   void launch_rhs(int k, hipStream_t st) const {
     for (const auto& G : ri.gs)
       hipLaunchKernelGGL(k_rhs_ib_jobs, dim3(G.nblk), dim3(64), 0, st, ri.djobs + G.job0[k], ri.dmap + G.map0);
@@ -1001,8 +1052,13 @@ struct IbSets {
     for (const auto& G : zf.gs)
       LH_DISPATCH_PLAN_SMALL(G.len, G.plan, launch_zfwd_jobs_t, double, st, zf.djobs + G.job0[k], zf.dmap + G.map0, G.nblk)
   }
+  void launch_plane(int k, hipStream_t st) const {
+    for (const auto& G : pl.gs)
+      LH_DISPATCH_IBP(G.len, G.plan, launch_ibp_t, st, pl.djobs + G.job0[k], G.nblk)
+  }
   void launch(int k, hipStream_t st) const {
     launch_rhs(k, st);
+    launch_plane(k, st);
     launch_zinv(k, st);
     launch_x(k, st);
     launch_zfwd(k, st);
@@ -1082,9 +1138,14 @@ static void issue_substep(lh_handle* h, int krk /*0-based*/, bool cfl_mode, int 
     const double z64 = 16.0 * dm.pz * dm.mx;
     const double nib = 2.0 * h->nibu + h->nibv;
     if (stages & kStageIBr) TIMED(h, LH_K_RHS, spl * 7.0 * nib, h->ib->launch_rhs(krk, h->st));
-    if (stages & kStageIBz) TIMED(h, LH_K_IBZ, (nib + 6.0) * (spl + z64), h->ib->launch_zinv(krk, h->st));
-    if (stages & kStageIBx) TIMED(h, LH_K_XIB, (2.0 * nib + 6.0) * z64, h->ib->launch_x(krk, h->st));
-    if (stages & kStageIBf) TIMED(h, LH_K_IBZ, nib * (spl + z64), h->ib->launch_zfwd(krk, h->st));
+    if (ib_plane(h)) {
+      // in: rhs of the canopy planes (and Lu_y of the tips); out: the forced rhs
+      if (stages & kStageIBz) TIMED(h, LH_K_XIB, (2.0 * nib + 12.0) * spl, h->ib->launch_plane(krk, h->st));
+    } else {
+      if (stages & kStageIBz) TIMED(h, LH_K_IBZ, (nib + 6.0) * (spl + z64), h->ib->launch_zinv(krk, h->st));
+      if (stages & kStageIBx) TIMED(h, LH_K_XIB, (2.0 * nib + 6.0) * z64, h->ib->launch_x(krk, h->st));
+      if (stages & kStageIBf) TIMED(h, LH_K_IBZ, nib * (spl + z64), h->ib->launch_zfwd(krk, h->st));
+    }
   } else if ((stages & kStageIB) && h->nibent > 0) {
     const int npl = h->nibu > h->nibv ? h->nibu : h->nibv;
     // in: u (3 rows), p, Nu_old, Nu_new per canopy plane; out: rhs (+ Lu_y of the tips)
@@ -1420,6 +1481,12 @@ int lh_create(const lh_config* c, lh_handle** out) {
     if (h->nibent > 0) {
       HIPCHK(h, hipMalloc((void**)&h->ibent, sizeof(IBEntry) * h->nibent));
       HIPCHK(h, hipMemcpy(h->ibent, ent.data(), sizeof(IBEntry) * h->nibent, hipMemcpyHostToDevice));
+      h->h_ent = ent;
+    }
+    if (ib_plane(h)) {
+      hipError_t ep = hipSuccess;
+      LH_DISPATCH_IBP(dm.px, dm.pz, attr_ibp_t, &ep)
+      HIPCHK(h, ep);
     }
     if (h->nibu) {
       HIPCHK(h, hipMalloc((void**)&h->ibu_planes, sizeof(int) * h->nibu));

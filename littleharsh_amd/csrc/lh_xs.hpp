@@ -216,9 +216,9 @@ template <> struct Family<96> : Two<96, 8, 12, 108, 2, 6> {};
 template <> struct Family<144> : Two<144, 12, 12, 156, 2, 6> {};
 template <> struct Family<384> : Whole384 {};
 
-// rows (z0, z0 + 1) at byte offset o of Z slot A -> X[t + T r] of their packed line in slot r (zero
-// past the kept modes)
-template <typename F> __device__ __forceinline__ void load(double2 (&v)[F::SL], const ColF& A, unsigned o, int t) {
+// rows (z0, z0 + 1) of a Z plane -> X[t + T r] of their packed line in slot r (zero past the kept
+// modes); get(row, mode) reads a row
+template <typename F, class Get> __device__ __forceinline__ void pack(double2 (&v)[F::SL], int t, Get get) {
   double2 a[F::R1], b[F::R1];
 #pragma unroll
   for (int r = 0; r < F::R1; ++r) {
@@ -226,8 +226,8 @@ template <typename F> __device__ __forceinline__ void load(double2 (&v)[F::SL], 
     if (first >= F::MX && last <= F::N - F::MX) continue;       // (decided when compiling)
     const int k = t + first;
     const int i = k < F::MX ? k : (k > F::N - F::MX ? F::N - k : 0);
-    a[r] = A.ld(o + (unsigned)i * 16u);
-    b[r] = A.ld(o + (unsigned)(F::MX + i) * 16u);
+    a[r] = get(0, i);
+    b[r] = get(1, i);
   }
 #pragma unroll
   for (int r = 0; r < F::R1; ++r) {
@@ -310,7 +310,10 @@ __global__ void __launch_bounds__(64 * xs::Family<N>::WPB) __attribute__((amdgpu
     for (int s = 0; s < SL; ++s) pk[64 * s] = x[s];
     xw::mem_fence_compiler();
   };
-  auto fetch = [&](C (&x)[SL], const C* z, int s) { xs::load<F>(x, ColF(z + (size_t)s * slot), o, t); };
+  auto fetch = [&](C (&x)[SL], const C* z, int s) {
+    const ColF A(z + (size_t)s * slot);
+    xs::pack<F>(x, t, [&](int row, int i) { return A.ld(o + (unsigned)(row * F::MX + i) * 16u); });
+  };
   auto out = [&](int q, int l, C (&x)[SL]) {
     F::fwd(x, t, buf, tw);
     if (st_ok) xs::store<F>(x, ColF(zp + ((size_t)q * nlev + l) * slot), o, t);
@@ -441,7 +444,8 @@ __global__ void __launch_bounds__(64 * xs::kSplitWaves) __attribute__((amdgpu_wa
   const C* zv = static_cast<const C*>(a.zv);
   const C* zp = static_cast<const C*>(a.zp);
   auto field = [&](C (&x)[SL], const C* z, int s) {
-    xs::load<F>(x, ColF(z + (size_t)s * slot), o, t);
+    const ColF A(z + (size_t)s * slot);
+    xs::pack<F>(x, t, [&](int row, int i) { return A.ld(o + (unsigned)(row * F::MX + i) * 16u); });
     F::inv(x, t, buf, tw);
   };
   auto out = [&](int q, C (&x)[SL]) {
