@@ -100,18 +100,59 @@ __global__ void __launch_bounds__(64) k_fwd(const uint16_t* __restrict__ X, cons
   }
 }
 
+// Adam on FP32 master parameter e with gradient ge (step t; bias corrections 1 - beta^t); refreshes
+// the bf16 copy of the weights
+struct Adam {
+  float *p, *m, *v;
+  uint16_t* wb;
+  const float* g;                             // gradients: parameter e's is g[e]
+  float lr, b1, b2, eps;
+  const float* part;                          // the step's loss: partial sums, over den
+  int nparts;
+  float den;
+  float* loss;
+};
+__device__ __forceinline__ void adam_step(const Adam& a, long long e, float ge, float t) {
+  const float c1 = 1.f - powf(a.b1, t), c2 = 1.f - powf(a.b2, t);
+  const float me = a.b1 * a.m[e] + (1.f - a.b1) * ge;
+  const float ve = a.b2 * a.v[e] + (1.f - a.b2) * ge * ge;
+  a.m[e] = me;
+  a.v[e] = ve;
+  const float pe = a.p[e] - a.lr * (me / c1) / (sqrtf(ve / c2) + a.eps);
+  a.p[e] = pe;
+  if (a.wb) a.wb[e] = f2bf(pe);
+}
+// the step's loss by a block's first 256 threads: fixed-order tree (every thread of the block calls)
+__device__ __forceinline__ void adam_loss(const Adam& a) {
+  __shared__ float red[256];
+  if (threadIdx.x < 256) {
+    float s = 0.f;
+    for (int i = threadIdx.x; i < a.nparts; i += 256) s += a.part[i];
+    red[threadIdx.x] = s;
+  }
+  __syncthreads();
+  for (int w = 128; w > 0; w >>= 1) {
+    if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) a.loss[0] = red[0] / a.den;
+}
+
 // dW = dZ^T X (dZ: B x N bf16, X: B x K bf16, dW: N x K f32), summed over the B rows; the
 // blocks of the extra last row (blockIdx.y = K / 16) form db = the column sums of the FP32 dZf
 // instead, beside the products.
 // One block of kDwWaves waves per 16x16 tile: wave w takes the row tiles w, w + kDwWaves, ...;
 // the partial tiles are summed in LDS in wave order (deterministic).
+// With ADAM the tile's owner also takes its parameters' step (t), the gradient still in hand: 15.5 us
+// at 4096 rows, as two launches 13.9 + 4.6 (sixteen row tiles' loads together: 17.7).
 constexpr int kDwWaves = 16;
+template <bool ADAM>
 __device__ __forceinline__ void dw_tile(const uint16_t* __restrict__ dZ, const uint16_t* __restrict__ X,
                                         float* __restrict__ dW, int B, int K, int N, const float* __restrict__ dZf,
-                                        float* __restrict__ db, int bx, int by) {
+                                        float* __restrict__ db, int bx, int by, const Adam& ad, float t) {
   __shared__ float part[kDwWaves][256];
   __shared__ float dbp[kDwWaves][64];
-  const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int l = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n0 = bx * 16, k0 = by * 16;
   if (k0 >= K) {                                    // bias row: column sums of dZf
     float sb = 0.f;
@@ -125,19 +166,30 @@ __device__ __forceinline__ void dw_tile(const uint16_t* __restrict__ dZ, const u
       for (int v = 0; v < kDwWaves; ++v)
         for (int gq = 0; gq < 4; ++gq) s += dbp[v][gq * 16 + threadIdx.x];
       db[n0 + threadIdx.x] = s;
+      if constexpr (ADAM) adam_step(ad, db + n0 + threadIdx.x - ad.g, s, t);
     }
     return;
   }
+  float* const d = dW + (size_t)(n0 + (threadIdx.x & 255) / 16) * K + k0 + threadIdx.x % 16;
   f4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (int r0 = 16 * w; r0 < B; r0 += 16 * kDwWaves) {
-    bf4 a, b;
+  // the row tiles w, w + kDwWaves, .. in order, the loads of U of them under way together
+  constexpr int U = 8;
+  const int nt = (B / 16 - w + kDwWaves - 1) / kDwWaves;
+  for (int i0 = 0; i0 < nt; i0 += U) {
+    bf4 a[U], b[U];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int r = r0 + 4 * (l / 16) + q;
-      a[q] = (short)dZ[(size_t)r * N + n0 + l % 16];   // A[i = neuron][k = row]
-      b[q] = (short)X[(size_t)r * K + k0 + l % 16];    // B[k = row][j = feature]
+    for (int u = 0; u < U; ++u) {
+      const int r0 = 16 * (w + kDwWaves * min(i0 + u, nt - 1));
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int r = r0 + 4 * (l / 16) + q;
+        a[u][q] = (short)dZ[(size_t)r * N + n0 + l % 16];   // A[i = neuron][k = row]
+        b[u][q] = (short)X[(size_t)r * K + k0 + l % 16];    // B[k = row][j = feature]
+      }
     }
-    acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (i0 + u < nt) acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[u], b[u], acc, 0, 0, 0);
   }
 #pragma unroll
   for (int q = 0; q < 4; ++q) part[w][(4 * (l / 16) + q) * 16 + l % 16] = acc[q];
@@ -145,19 +197,21 @@ __device__ __forceinline__ void dw_tile(const uint16_t* __restrict__ dZ, const u
   if (threadIdx.x < 256) {
     float s = 0.f;
     for (int v = 0; v < kDwWaves; ++v) s += part[v][threadIdx.x];
-    dW[(size_t)(n0 + threadIdx.x / 16) * K + k0 + threadIdx.x % 16] = s;
+    *d = s;
+    if constexpr (ADAM) adam_step(ad, d - ad.g, s, t);
   }
 }
 __global__ void __launch_bounds__(64 * kDwWaves) k_dw(const uint16_t* __restrict__ dZ,
                                                       const uint16_t* __restrict__ X,
                                                       float* __restrict__ dW, int B, int K, int N,
                                                       const float* __restrict__ dZf, float* __restrict__ db) {
-  dw_tile(dZ, X, dW, B, K, N, dZf, db, blockIdx.x, blockIdx.y);
+  dw_tile<false>(dZ, X, dW, B, K, N, dZf, db, blockIdx.x, blockIdx.y, Adam{}, 0.f);
 }
 
 // The weight gradients of every layer in one launch: block b of layer l is the block
-// (b % (N / 16), b / (N / 16)) of that layer's k_dw grid.  With tstep, block 0 advances the
-// step counter (the step's gather has finished and no block here reads it).
+// (b % (N / 16), b / (N / 16)) of that layer's k_dw grid.  With ADAM also the step of every
+// parameter, each by the thread that holds its gradient; one more block forms the step's loss and
+// makes tstep[1], the step (k_train_s set it), the count of steps taken (nothing here reads tstep[0]).
 constexpr int kMaxL = 8;
 struct DwAll {
   const uint16_t* dZ[kMaxL];
@@ -169,12 +223,18 @@ struct DwAll {
   int L, B;
   int* tstep;
 };
-__global__ void __launch_bounds__(64 * kDwWaves) k_dw_all(DwAll a) {
+template <bool ADAM>
+__global__ void __launch_bounds__(64 * kDwWaves) k_dw_all(DwAll a, Adam ad) {
+  const int step = ADAM ? a.tstep[1] : 0;
+  if (ADAM && (int)blockIdx.x == a.first[a.L]) {
+    adam_loss(ad);
+    if (threadIdx.x == 0) a.tstep[0] = step;
+    return;
+  }
   int l = 0;
   while (l + 1 < a.L && (int)blockIdx.x >= a.first[l + 1]) ++l;
   const int b = blockIdx.x - a.first[l], nbx = a.N[l] / 16;
-  dw_tile(a.dZ[l], a.X[l], a.dW[l], a.B, a.K[l], a.N[l], a.dZf[l], a.db[l], b % nbx, b / nbx);
-  if (a.tstep && blockIdx.x == 0 && threadIdx.x == 0) a.tstep[0] = a.tstep[0] + 1;
+  dw_tile<ADAM>(a.dZ[l], a.X[l], a.dW[l], a.B, a.K[l], a.N[l], a.dZf[l], a.db[l], b % nbx, b / nbx, ad, (float)step);
 }
 
 // the previous layer's dZ = (dZ W) * (1 - tanh(Zp)^2) (dZ: B x N bf16, W: N x K bf16, Zp: its
@@ -253,6 +313,10 @@ __global__ void __launch_bounds__(256) k_mse(const float* __restrict__ Y, const 
 // wave's tile) in registers: the input-gradient epilogue of the same tile reads them in the
 // same lanes.  Layer inputs and dZ pass between layers through ping-pong LDS tiles (one
 // barrier per layer) and go to global memory for the weight gradients (k_dw_all).
+// row of the data set that row r of step's batch is
+__device__ __forceinline__ long long draw_row(uint64_t seed, uint64_t step, int r, long long n) {
+  return (long long)(mix64(seed ^ mix64(step * 0x100000001b3ull + (uint64_t)r)) % (uint64_t)n);
+}
 struct TrainNet {
   const uint16_t* w[kMaxL];   // bf16 weights of each layer (N x K)
   const float* b[kMaxL];      // FP32 biases
@@ -262,8 +326,18 @@ struct TrainNet {
   const float* T;             // targets (B x nout)
   float* part;                // loss partial sums, one per 16-row tile
   int B, nout;
+  // a batch drawn from a data set (k_gather's rows): X[0] is written then, and T not used
+  const float *x, *y;
+  long long n;
+  int nin;
+  uint64_t seed;
+  int* tstep;                 // [0] steps taken, [1] the step under way, set here
 };
-template <int K0, int NH, int NHH>
+// GATHER: the block draws its own 16 rows (a wave a row at a time) into LDS, its first layer's
+// operand, and into X[0] for the weight gradients.  Bound by the chain of layers, one wave per SIMD:
+// 17.6 us at 4096 rows, where drawing the rows in a launch of their own and fetching each layer's
+// weights behind its barrier took 6.1 + 12.7 us.
+template <int K0, int NH, int NHH, bool GATHER>
 __global__ void __launch_bounds__(4 * NH) k_train_s(TrainNet tn) {
   static_assert(K0 % 32 == 0 && NH % 32 == 0, "32-wide forward steps without a tail");
   constexpr int L = NHH + 2, NO = 16;
@@ -273,21 +347,70 @@ __global__ void __launch_bounds__(4 * NH) k_train_s(TrainNet tn) {
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63, li = l & 15, lg = l >> 4;
   const int b0 = blockIdx.x * 16, col = w * 16 + li;
   f4 zr[NHH + 1];                                      // this wave's hidden pre-activations
+  // every weight and bias of the wave's tiles, fetched together ahead of the chain of layers
+  bf8 w0[K0 / 32], wf[NHH][NH / 32], wo[NH / 32];      // forward: rows of W
+  bf4 wb[NHH][NH / 16], wbo;                           // input gradients: columns of W
+  float bh[NHH + 1];
+#pragma unroll
+  for (int c = 0; c < K0 / 32; ++c) w0[c] = ld8(tn.w[0] + (size_t)col * K0 + c * 32 + 8 * lg);
+#pragma unroll
+  for (int h = 0; h < NHH; ++h) {
+#pragma unroll
+    for (int c = 0; c < NH / 32; ++c) wf[h][c] = ld8(tn.w[h + 1] + (size_t)col * NH + c * 32 + 8 * lg);
+#pragma unroll
+    for (int c = 0; c < NH / 16; ++c)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) wb[h][c][q] = (short)tn.w[h + 1][(size_t)(16 * c + 4 * lg + q) * NH + col];
+  }
+#pragma unroll
+  for (int c = 0; c < NH / 32; ++c) wo[c] = ld8(tn.w[L - 1] + (size_t)li * NH + c * 32 + 8 * lg);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) wbo[q] = (short)tn.w[L - 1][(size_t)(4 * lg + q) * NH + col];
+#pragma unroll
+  for (int h = 0; h <= NHH; ++h) bh[h] = tn.b[h][col];
+  const float bo = tn.b[L - 1][li];
+  constexpr int XS = K0 + 8;                           // (row stride: 16 bytes past a multiple of the banks)
+  __shared__ __align__(16) uint16_t x0[GATHER ? 16 * XS : 8];
+  __shared__ float tg[GATHER ? 256 : 1];               // targets of the rows
+  if constexpr (GATHER) {
+    const uint64_t step = (uint64_t)tn.tstep[0];
+    if (blockIdx.x == 0 && threadIdx.x == 0) tn.tstep[1] = (int)step + 1;
+    constexpr int RW = 16 / (NH / 16), NF = K0 / 64;   // rows per wave, values of a row per lane
+    float v[RW][NF], tv[RW];
+    const long long mine = draw_row(tn.seed, step, b0 + w * RW + l % RW, tn.n);     // (one division a lane)
+#pragma unroll
+    for (int i = 0; i < RW; ++i) {
+      const long long src = __shfl(mine, i, 64);
+#pragma unroll
+      for (int c = 0; c < NF; ++c) v[i][c] = l + 64 * c < tn.nin ? tn.x[(size_t)src * tn.nin + l + 64 * c] : 0.f;
+      tv[i] = l < tn.nout ? tn.y[(size_t)src * tn.nout + l] : 0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < RW; ++i) {
+      const int r = w * RW + i;
+#pragma unroll
+      for (int c = 0; c < NF; ++c) {
+        const uint16_t x = l + 64 * c < tn.nin ? f2bf(v[i][c]) : (uint16_t)0;
+        x0[r * XS + l + 64 * c] = x;
+        tn.X[0][(size_t)(b0 + r) * K0 + l + 64 * c] = x;
+      }
+      if (l < 16) tg[r * 16 + l] = tv[i];
+    }
+    __syncthreads();
+  }
   {
-    const uint16_t* xr = tn.X[0] + (size_t)(b0 + li) * K0;
-    const uint16_t* wr = tn.w[0] + (size_t)col * K0;
+    const uint16_t* xr = GATHER ? x0 + li * XS : tn.X[0] + (size_t)(b0 + li) * K0;
     f4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int k0 = 0; k0 < K0; k0 += 32) acc = mfma32(ld8(xr + k0 + 8 * lg), ld8(wr + k0 + 8 * lg), acc);
+    for (int k0 = 0; k0 < K0; k0 += 32) acc = mfma32(ld8(xr + k0 + 8 * lg), w0[k0 / 32], acc);
     zr[0] = acc;
   }
 #pragma unroll
   for (int h = 0; h <= NHH; ++h) {
     uint16_t* xo = xt[(h + 1) & 1];
-    const float bb = tn.b[h][col];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      const float z = zr[h][q] + bb;
+      const float z = zr[h][q] + bh[h];
       zr[h][q] = z;
       const uint16_t x = f2bf(tanh_act(z));
       xo[(4 * lg + q) * NH + col] = x;
@@ -298,18 +421,15 @@ __global__ void __launch_bounds__(4 * NH) k_train_s(TrainNet tn) {
 #pragma unroll
     for (int c = 0; c < NH / 32; ++c) a[c] = ld8(xo + li * NH + c * 32 + 8 * lg);
     if (h < NHH) {
-      const uint16_t* wr = tn.w[h + 1] + (size_t)col * NH;
       f4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int c = 0; c < NH / 32; ++c) acc = mfma32(a[c], ld8(wr + c * 32 + 8 * lg), acc);
+      for (int c = 0; c < NH / 32; ++c) acc = mfma32(a[c], wf[h][c], acc);
       zr[h + 1] = acc;
     } else if (w == 0) {
       // output layer and the loss terms
-      const uint16_t* wr = tn.w[L - 1] + (size_t)li * NH;
       f4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int c = 0; c < NH / 32; ++c) acc = mfma32(a[c], ld8(wr + c * 32 + 8 * lg), acc);
-      const float bo = tn.b[L - 1][li];
+      for (int c = 0; c < NH / 32; ++c) acc = mfma32(a[c], wo[c], acc);
       const float sc = 2.f / (float)(tn.B * tn.nout);
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
@@ -317,7 +437,7 @@ __global__ void __launch_bounds__(4 * NH) k_train_s(TrainNet tn) {
         const float y = acc[q] + bo;
         float d = 0.f, s = 0.f;
         if (li < tn.nout) {
-          d = y - tn.T[(size_t)r * tn.nout + li];
+          d = y - (GATHER ? tg[(4 * lg + q) * 16 + li] : tn.T[(size_t)r * tn.nout + li]);
           s = d * d;
         }
         const size_t o = (size_t)r * NO + li;
@@ -350,14 +470,11 @@ __global__ void __launch_bounds__(4 * NH) k_train_s(TrainNet tn) {
 #pragma unroll
     for (int n0 = 0; n0 < NH; n0 += 16)
       if (n0 < N) a[n0 / 16] = *reinterpret_cast<const bf4*>(src + li * N + n0 + 4 * lg);
-    const uint16_t* W = tn.w[ly];
     f4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int n0 = 0; n0 < NH; n0 += 16) {
       if (n0 < N) {
-        bf4 b;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) b[q] = (short)W[(size_t)(n0 + 4 * lg + q) * K + col];
+        const bf4 b = ly == L - 1 ? wbo : wb[ly == L - 1 ? 0 : ly - 1][n0 / 16];
         acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[n0 / 16], b, acc, 0, 0, 0);
       }
     }
@@ -393,7 +510,7 @@ __global__ void k_gather(const float* __restrict__ x, const float* __restrict__ 
   const int r = blockIdx.x;
   if (r >= B) return;
   const uint64_t step = (uint64_t)tstep[0];
-  const long long src = (long long)(mix64(seed ^ mix64(step * 0x100000001b3ull + (uint64_t)r)) % (uint64_t)n);
+  const long long src = draw_row(seed, step, r, n);
   for (int f = threadIdx.x; f < K0; f += blockDim.x)
     X[(size_t)r * K0 + f] = f < nin ? f2bf(x[(size_t)src * nin + f]) : (uint16_t)0;
   for (int f = threadIdx.x; f < nout; f += blockDim.x) T[(size_t)r * nout + f] = y[(size_t)src * nout + f];
@@ -756,37 +873,11 @@ __global__ void k_unpack_out(const float* __restrict__ Z, int NP, int nout, int 
   if (e < nrow * nout) y[e] = Z[(size_t)(e / nout) * NP + e % nout];
 }
 
-// Adam on the FP32 master parameters (step t = tstep, already advanced by k_mse; bias
-// corrections 1 - beta^t); refreshes the bf16 copy of the weights; the first thread also sums
-// the step's loss
-__global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
-                       float* __restrict__ v, uint16_t* __restrict__ wb, long long n, float lr, float b1, float b2,
-                       float eps, const int* __restrict__ tstep, const float* __restrict__ part, int nparts,
-                       float den, float* __restrict__ loss) {
+// every parameter's Adam step (step t = tstep, already advanced by k_mse) and the step's loss
+__global__ void k_adam(Adam a, long long n, const int* __restrict__ tstep) {
   const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (blockIdx.x == 0) {                            // the step's loss: fixed-order tree
-    __shared__ float red[256];
-    float s = 0.f;
-    for (int i = threadIdx.x; i < nparts; i += 256) s += part[i];
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-      if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) loss[0] = red[0] / den;
-  }
-  if (e >= n) return;
-  const float t = (float)tstep[0];
-  const float c1 = 1.f - powf(b1, t), c2 = 1.f - powf(b2, t);
-  const float ge = g[e];
-  const float me = b1 * m[e] + (1.f - b1) * ge;
-  const float ve = b2 * v[e] + (1.f - b2) * ge * ge;
-  m[e] = me;
-  v[e] = ve;
-  const float pe = p[e] - lr * (me / c1) / (sqrtf(ve / c2) + eps);
-  p[e] = pe;
-  if (wb) wb[e] = f2bf(pe);
+  if (blockIdx.x == 0) adam_loss(a);
+  if (e < n) adam_step(a, e, a.g[e], (float)tstep[0]);
 }
 
 __global__ void k_to_bf(const float* __restrict__ p, uint16_t* __restrict__ wb, long long n) {
@@ -895,10 +986,15 @@ static void mlp_backward(lh_mlp* h) {
   }
 }
 
+static Adam adam_args(lh_mlp* h, float lr) {
+  return Adam{h->p, h->m, h->v, h->wb, h->g, lr, 0.9f, 0.999f, 1e-8f, h->part, h->nparts, (float)(h->B * h->nout), h->loss};
+}
+
 // the closure network's shape: forward, loss terms and input gradients of the batch in X[0]
-// (k_train_s), then every layer's weight gradients (k_dw_all); with tick, the step counter
-// advances.  The same results as mlp_forward + mlp_loss + mlp_backward, in two launches.
-static void spec_pass(lh_mlp* h, bool tick) {
+// (k_train_s), then every layer's weight gradients (k_dw_all).  The same results as mlp_forward +
+// mlp_loss + mlp_backward, in two launches; with train, a whole step in the same two: the batch is
+// drawn in the first and the parameters take their step in the second.
+static void spec_pass(lh_mlp* h, bool train, float lr = 0.f, uint64_t seed = 0) {
   TrainNet tn{};
   DwAll a{};
   int nb = 0;
@@ -921,13 +1017,24 @@ static void spec_pass(lh_mlp* h, bool tick) {
   a.first[h->L] = nb;
   a.L = h->L;
   a.B = h->B;
-  a.tstep = tick ? h->tdev : nullptr;
+  a.tstep = h->tdev;
   tn.T = h->T;
   tn.part = h->part;
   tn.B = h->B;
   tn.nout = h->nout;
-  hipLaunchKernelGGL((k_train_s<256, 64, 3>), dim3(h->B / 16), dim3(4 * 64), 0, h->st, tn);
-  hipLaunchKernelGGL(k_dw_all, dim3(nb), dim3(64 * kDwWaves), 0, h->st, a);
+  if (train) {
+    tn.x = h->dx;
+    tn.y = h->dy;
+    tn.n = h->ndata;
+    tn.nin = h->nin;
+    tn.seed = seed;
+    tn.tstep = h->tdev;
+    hipLaunchKernelGGL((k_train_s<256, 64, 3, true>), dim3(h->B / 16), dim3(4 * 64), 0, h->st, tn);
+    hipLaunchKernelGGL(k_dw_all<true>, dim3(nb + 1), dim3(64 * kDwWaves), 0, h->st, a, adam_args(h, lr));
+  } else {
+    hipLaunchKernelGGL((k_train_s<256, 64, 3, false>), dim3(h->B / 16), dim3(4 * 64), 0, h->st, tn);
+    hipLaunchKernelGGL(k_dw_all<false>, dim3(nb), dim3(64 * kDwWaves), 0, h->st, a, Adam{});
+  }
 }
 
 extern "C" {
@@ -1111,19 +1218,17 @@ int lh_mlp_loss_grad(lh_mlp* h, const float* x, const float* y, float* loss, flo
 // one Adam step on a batch drawn from the data set; the step count lives on the device, so
 // the same launches (captured once as a graph) serve every step
 static void issue_train_step(lh_mlp* h, float lr, unsigned long long seed) {
-  const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
+  if (h->spec && h->fused) {
+    spec_pass(h, true, lr, seed);
+    return;
+  }
   hipLaunchKernelGGL(k_gather, dim3(h->B), dim3(64), 0, h->st, h->dx, h->dy, h->ndata, h->nin, h->nout,
                      h->Kp[0], h->B, (uint64_t)seed, (const int*)h->tdev, h->X[0], h->T);
-  if (h->spec && h->fused) {
-    spec_pass(h, true);
-  } else {
-    mlp_forward(h);
-    mlp_loss(h, true);
-    mlp_backward(h);
-  }
-  hipLaunchKernelGGL(k_adam, dim3((unsigned)((h->np + 255) / 256)), dim3(256), 0, h->st, h->p, h->g, h->m,
-                     h->v, h->wb, h->np, lr, b1, b2, eps, (const int*)h->tdev, h->part, h->nparts,
-                     (float)(h->B * h->nout), h->loss);
+  mlp_forward(h);
+  mlp_loss(h, true);
+  mlp_backward(h);
+  hipLaunchKernelGGL(k_adam, dim3((unsigned)((h->np + 255) / 256)), dim3(256), 0, h->st, adam_args(h, lr),
+                     (long long)h->np, (const int*)h->tdev);
 }
 
 // captures `n` consecutive training steps as one graph
