@@ -1308,8 +1308,9 @@ int lh_create(const lh_config* c, lh_handle** out) {
     if (h->xraw_lc <= 0) h->xraw_lc = chunk_levels(dm.nyu - 2, dm.pz / 2, ncu * bx, 4, 64, 1.0);
     // the wave assembly: one block per CU; a chunk's start-up is half a level (three tiles of six)
     if (h->zasm_lc <= 0 && use_zw(h)) h->zasm_lc = chunk_levels(dm.nyu - 2, zw::groups(dm.mx), ncu, 2, 96, 0.5);
+    // (one level per block where all of them are resident: 8.2 against 10.2 us at 32 x 41 x 32)
     if (h->zasm_lc <= 0)
-      h->zasm_lc = chunk_levels(dm.nyu - 2, 3L * ((dm.mx + LH_ZASM_COLS - 1) / LH_ZASM_COLS), ncu * bz, 2, 12, 0.25);
+      h->zasm_lc = chunk_levels(dm.nyu - 2, 3L * ((dm.mx + LH_ZASM_COLS - 1) / LH_ZASM_COLS), ncu * bz, 1, 12, 0.25);
   }
   const size_t nu = (size_t)dm.nyu * dm.ncol, nv = (size_t)dm.nyv * dm.ncol,
                np = (size_t)dm.nyp * dm.ncol;
