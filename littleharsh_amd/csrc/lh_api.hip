@@ -5,8 +5,8 @@
 //   NL stage   : k_zinv (u,w,v) -> k_xw576 at 576 points in x, k_xs (k_xraw2 in mixed
 //                precision) at the other sizes
 //                (x transforms, six products, CFL max)
-//                -> k_zasm (A/B recombination, forward z transforms -> Nu_new), k_zw576 for FP64
-//                planes of 576 x 576 points
+//                -> k_zasm (A/B recombination, forward z transforms -> Nu_new), k_zw for FP64
+//                planes of 576 x 576 and of 384 x 384 points
 //   IB stage   : k_rhs_ib (rhs and Lu_y on canopy planes), then k_ib_plane (FP64, lengths up to
 //                144) or k_zinv -> k_xpass_ib -> k_zfwd
 //   column     : k_prep (LU of the shared velocity matrices) -> k_col (RHS0 + rhs of solveU/V,
@@ -324,10 +324,13 @@ static void launch_xraw_t(lh_handle* h, const XRAW& a, const void* tw) {
 #endif
 template <typename TR> struct XwWaves { static constexpr int value = sizeof(TR) == 8 ? 8 : LH_XW_WAVES32; };
 static bool use_xw(const lh_handle* h) { return h->dm.px == 576; }
-// products in tiles and the one-wave-per-line z assembly: FP64 planes of 576 x 576 points, whose z
-// lines are the waves' 576-point transform (per substep of 384 x 289 x 384, x pass and assembly: 2.09
-// ms, with rows and k_zasm 2.77).  Mixed precision keeps k_zasm's operation order
-static bool use_zw(const lh_handle* h) { return use_xw(h) && h->dm.pz == zw::N && h->prec == LH_PREC_FP64; }
+// products in tiles and the one-wave-per-line z assembly: square FP64 planes of 384 or 576 points,
+// whose z lines fill a wave (per substep, x pass and assembly: 384 x 289 x 384 2.09 ms, with rows and
+// k_zasm 2.77; 256 x 97 x 256 0.36 against 0.49).  Shorter lines leave k_zasm's shape: 96 x 145 x 96
+// reads 0.1 GB in 36 us.  Mixed precision keeps k_zasm's operation order
+static bool use_zw(const lh_handle* h) {
+  return h->prec == LH_PREC_FP64 && h->dm.px == h->dm.pz && (h->dm.pz == 576 || h->dm.pz == 384);
+}
 template <typename TR>
 static void launch_xw_t(lh_handle* h, int want_cfl) {
   XW a{h->zu, h->zw, h->zv, h->zp, sizeof(TR) == 8 ? (const void*)h->twxw : (const void*)h->twxw32,
@@ -368,6 +371,15 @@ template <int N> static void launch_xs_t(lh_handle* h, int want_cfl) {
   using F = xs::Family<N>;
   XW a{h->zu, h->zw, h->zv, h->zp, h->twx, h->dthdyu, h->scal, want_cfl, h->xraw_lc};
   const long groups = (h->dm.pz / 2 + F::LPW - 1) / F::LPW, nlev = h->dm.nyu - 2;
+  if constexpr (F::LPW == 1) {
+    if (use_zw(h)) {
+      const long waves = groups * ((nlev + a.lc - 1) / a.lc);
+      const dim3 grid((unsigned)((waves + F::WPB - 1) / F::WPB)), block(64 * F::WPB);
+      if (want_cfl) hipLaunchKernelGGL((k_xs<N, true, true>), grid, block, xs::lds_bytes<F>(), h->st, a, h->dm);
+      else hipLaunchKernelGGL((k_xs<N, false, true>), grid, block, xs::lds_bytes<F>(), h->st, a, h->dm);
+      return;
+    }
+  }
   if (a.lc == 1 && xs::kSplitWaves * groups * nlev <= 8L * h->ncu) {
     const dim3 grid((unsigned)(groups * nlev)), block(64 * xs::kSplitWaves);
     if (want_cfl) hipLaunchKernelGGL((k_xs_split<N, true>), grid, block, xs::split_lds_bytes<F>(), h->st, a, h->dm);
@@ -376,8 +388,8 @@ template <int N> static void launch_xs_t(lh_handle* h, int want_cfl) {
   }
   const long waves = groups * ((nlev + a.lc - 1) / a.lc);
   const dim3 grid((unsigned)((waves + F::WPB - 1) / F::WPB)), block(64 * F::WPB);
-  if (want_cfl) hipLaunchKernelGGL((k_xs<N, true>), grid, block, xs::lds_bytes<F>(), h->st, a, h->dm);
-  else hipLaunchKernelGGL((k_xs<N, false>), grid, block, xs::lds_bytes<F>(), h->st, a, h->dm);
+  if (want_cfl) hipLaunchKernelGGL((k_xs<N, true, false>), grid, block, xs::lds_bytes<F>(), h->st, a, h->dm);
+  else hipLaunchKernelGGL((k_xs<N, false, false>), grid, block, xs::lds_bytes<F>(), h->st, a, h->dm);
 }
 static hipError_t max_lds(const void* kernel, size_t bytes) {
   return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
@@ -390,8 +402,12 @@ static hipError_t attr_xw_t() {
 }
 template <int N> static void attr_xs_t(hipError_t* e) {
   constexpr size_t sh = xs::lds_bytes<xs::Family<N>>();
-  *e = max_lds((const void*)k_xs<N, true>, sh);
-  if (*e == hipSuccess) *e = max_lds((const void*)k_xs<N, false>, sh);
+  *e = max_lds((const void*)k_xs<N, true, false>, sh);
+  if (*e == hipSuccess) *e = max_lds((const void*)k_xs<N, false, false>, sh);
+  if constexpr (xs::Family<N>::LPW == 1) {
+    if (*e == hipSuccess) *e = max_lds((const void*)k_xs<N, true, true>, sh);
+    if (*e == hipSuccess) *e = max_lds((const void*)k_xs<N, false, true>, sh);
+  }
   constexpr size_t sp = xs::split_lds_bytes<xs::Family<N>>();
   static_assert(sp <= 64 * 1024, "within the default limit");
 }
@@ -403,9 +419,10 @@ template <int N> static void xs_levels_t(lh_handle* h, int ncu) {
 }
 static void launch_zw(lh_handle* h, const ZASM& z) {
   const Dims& dm = h->dm;
-  ZW a{(const double2*)h->zp, h->twxw, z.nu1, z.nu2, z.nu3, z.dthdyu, z.dthdyv, z.k1x, z.k1z, z.lc, z.prep, z.cfl};
+  ZW a{(const double2*)h->zp, (const double2*)h->twz64, z.nu1, z.nu2, z.nu3, z.dthdyu, z.dthdyv, z.k1x, z.k1z, z.lc, z.prep, z.cfl};
   const int nb = zw::groups(dm.mx) * ((dm.nyu - 2 + a.lc - 1) / a.lc) + (a.prep ? kPrepBlocks : 0);
-  hipLaunchKernelGGL(k_zw576, dim3(nb), dim3(512), zw::lds_bytes(), h->st, a, dm);
+  if (dm.pz == 576) hipLaunchKernelGGL(k_zw<576>, dim3(nb), dim3(512), zw::Shape<576>::LDS, h->st, a, dm);
+  else hipLaunchKernelGGL(k_zw<384>, dim3(nb), dim3(512), zw::Shape<384>::LDS, h->st, a, dm);
 }
 // the canopy x pass at 576 points: one wave per (entry, row pair), LH_XIBW_WAVES per block
 // (12: three per SIMD at 132 VGPRs, 121 KB of LDS; 16 would spill)
@@ -1292,7 +1309,6 @@ int lh_create(const lh_config* c, lh_handle** out) {
       const bool f64 = h->prec == LH_PREC_FP64;
       const hipError_t ea = !f64 ? attr_xw_t<float, false>() : (use_zw(h) ? attr_xw_t<double, true>() : attr_xw_t<double, false>());
       HIPCHK(h, ea);
-      if (use_zw(h)) HIPCHK(h, max_lds((const void*)k_zw576, zw::lds_bytes()));
       HIPCHK(h, hipFuncSetAttribute((const void*)k_xpass_ib576<LH_XIBW_WAVES>,
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)xibw_lds_bytes()));
       const int wpb = f64 ? XwWaves<double>::value : XwWaves<float>::value;
@@ -1306,6 +1322,10 @@ int lh_create(const lh_config* c, lh_handle** out) {
       if (h->xraw_lc <= 0) LH_DISPATCH_XS(dm.px, xs_levels_t, h, ncu)
     }
     if (h->xraw_lc <= 0) h->xraw_lc = chunk_levels(dm.nyu - 2, dm.pz / 2, ncu * bx, 4, 64, 1.0);
+    if (use_zw(h)) {
+      HIPCHK(h, max_lds((const void*)k_zw<576>, zw::Shape<576>::LDS));
+      HIPCHK(h, max_lds((const void*)k_zw<384>, zw::Shape<384>::LDS));
+    }
     // the wave assembly: one block per CU; a chunk's start-up is half a level (three tiles of six)
     if (h->zasm_lc <= 0 && use_zw(h)) h->zasm_lc = chunk_levels(dm.nyu - 2, zw::groups(dm.mx), ncu, 2, 96, 0.5);
     // (one level per block where all of them are resident: 8.2 against 10.2 us at 32 x 41 x 32)
@@ -1355,7 +1375,7 @@ int lh_create(const lh_config* c, lh_handle** out) {
   HIPCHK(h, hipMalloc(&h->zv, zel * zslot * dm.nyv));
   // zp also serves as the FP64 scratch of the IB stage
   {
-    size_t nzp = use_zw(h) ? zel * zw::zp_values(nlev, dm.mx) : zel * zslot * 6 * (size_t)nlev;
+    size_t nzp = use_zw(h) ? zel * zw::zp_values(nlev, dm.mx, dm.pz) : zel * zslot * 6 * (size_t)nlev;
     size_t nib = sizeof(double2) * zslot * (3 * (size_t)dm.nyu + 6);
     HIPCHK(h, hipMalloc(&h->zp, nzp > nib ? nzp : nib));
   }

@@ -258,6 +258,17 @@ template <typename F> __device__ __forceinline__ void store(const double2 (&v)[F
   }
 }
 
+// the same as one row pair of the product tiles of lh_zw.hpp (as xw::store_tile), group values apart
+template <typename F>
+__device__ __forceinline__ void store_tile(const double2 (&v)[F::SL], const ColF& d, int group, int t) {
+#pragma unroll
+  for (int r = 0; r < F::R1; ++r) {
+    const int k = t + F::T * r, m = F::N - k;
+    if (k < F::MX) d.st_nt((unsigned)((k >> 3) * group + (k & 7)) * 16u, v[r]);
+    else if (m < F::MX) d.st_nt((unsigned)((m >> 3) * group + 8 + (m & 7)) * 16u, v[r]);
+  }
+}
+
 constexpr int kSplitWaves = 3;
 template <typename F> constexpr size_t split_lds_bytes() {
   return sizeof(double2) * ((size_t)F::TWN + (size_t)kSplitWaves * F::LINE);
@@ -270,10 +281,12 @@ template <typename F> constexpr size_t lds_bytes() {
 
 // One wave per (F::LPW row pairs, chunk of lc levels); the walk over the levels, the fields carried
 // and the park line are those of k_xw576.
-template <int N, bool CFL>
+// TILE (one line per wave): rows z and z + pz / 2 pair up and the products go out in tiles
+template <int N, bool CFL, bool TILE>
 __global__ void __launch_bounds__(64 * xs::Family<N>::WPB) __attribute__((amdgpu_waves_per_eu(2)))
     k_xs(XW a, Dims dm) {
   using F = xs::Family<N>;
+  static_assert(!TILE || F::LPW == 1, "tiles: the row pair is the wave's");
   using C = double2;
   constexpr int SL = F::SL;
   extern __shared__ char smem_raw[];
@@ -295,7 +308,8 @@ __global__ void __launch_bounds__(64 * xs::Family<N>::WPB) __attribute__((amdgpu
   if (l0 >= l1) return;
   const int pr = (item % nwc) * F::LPW + ln;
   const bool st_ok = pr < npair && lane < F::LPW * F::T;
-  const unsigned o = (unsigned)min(pr, npair - 1) * (unsigned)(2 * F::MX * sizeof(C));
+  const unsigned o = (unsigned)min(pr, npair - 1) * (unsigned)((TILE ? 1 : 2) * F::MX * sizeof(C));
+  const int second = TILE ? npair * F::MX : F::MX;              // from a pair's first row to its second
   const size_t slot = (size_t)dm.pz * F::MX;
   const C* zu = static_cast<const C*>(a.zu);
   const C* zw = static_cast<const C*>(a.zw);
@@ -312,11 +326,16 @@ __global__ void __launch_bounds__(64 * xs::Family<N>::WPB) __attribute__((amdgpu
   };
   auto fetch = [&](C (&x)[SL], const C* z, int s) {
     const ColF A(z + (size_t)s * slot);
-    xs::pack<F>(x, t, [&](int row, int i) { return A.ld(o + (unsigned)(row * F::MX + i) * 16u); });
+    xs::pack<F>(x, t, [&](int row, int i) { return A.ld(o + (unsigned)(row * second + i) * 16u); });
   };
   auto out = [&](int q, int l, C (&x)[SL]) {
     F::fwd(x, t, buf, tw);
-    if (st_ok) xs::store<F>(x, ColF(zp + ((size_t)q * nlev + l) * slot), o, t);
+    if constexpr (TILE) {
+      const int group = (npair + 1) * 16;
+      xs::store_tile<F>(x, ColF(zp + ((size_t)q * nlev + l) * ((F::MX + 7) / 8) * group + pr * 16), group, t);
+    } else {
+      if (st_ok) xs::store<F>(x, ColF(zp + ((size_t)q * nlev + l) * slot), o, t);
+    }
   };
   fetch(cu, zu, l0 + 1);
   if constexpr (!F::EARLY) F::inv(cu, t, buf, tw);
