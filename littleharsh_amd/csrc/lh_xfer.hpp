@@ -119,13 +119,15 @@ inline hipError_t xfer_bytes(bool up, int dev, hipStream_t st, char* stage, cons
     }
   }
   // chunk k of the job: up to kChunk bytes of one field
-  size_t first[6] = {0};
+  size_t first[6] = {0}, total = 0;
   for (int i = 0; i < nf; ++i) {
     const size_t bytes = fs.f[i].host ? (size_t)fs.f[i].n * ncol * el : 0;
+    total += bytes;
     first[i + 1] = first[i] + (bytes + HostStage::kChunk - 1) / HostStage::kChunk;
   }
   const size_t nchunk = first[nf];
-  const int nt = (int)std::min<size_t>(HostStage::kThreads, std::max<size_t>(1, nchunk));
+  // (a thread per chunk's worth of bytes: below that its start costs more than the copy it takes over)
+  const int nt = (int)std::min<size_t>(HostStage::kThreads, 1 + total / HostStage::kChunk);
   std::atomic<size_t> next{0};
   std::atomic<int> err{(int)hipSuccess};
   auto work = [&](int t) {
