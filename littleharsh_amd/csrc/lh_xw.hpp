@@ -1,7 +1,8 @@
 // lh_xw.hpp -- the nonlinear x pass with one wavefront per 576-point line (gfx950; FP64, and
 // FP32 for the transforms of the mixed-precision mode).
 //
-// Each wave owns one row pair (z0, z0+1) of the Z slots and walks up a chunk of levels, as
+// Each wave owns one row pair ((z0, z0+1), or (z, z + 288) for the tiles of lh_zw.hpp) of the Z slots
+// and walks up a chunk of levels, as
 // the block-level pass k_xraw2 does, but every 576-point transform is done by that wave
 // alone: 9 points per lane, no workgroup barrier.  576 = 9 x 64:
 //
