@@ -163,9 +163,9 @@ class DeviceClosure:
         self._check(self.lib.lh_closure_apply(self.h), "lh_closure_apply")
 
     def close(self):
-        if self.h:
-            self.lib.lh_closure_destroy(self.h)
-            self.h = ctypes.c_void_p()
+        h, self.h = self.h, None
+        if h:
+            self.lib.lh_closure_destroy(h)
 
     def __del__(self):
         try:

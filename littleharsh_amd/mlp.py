@@ -47,9 +47,9 @@ class MLP:
             raise RuntimeError(f"{what}: status {st}: {msg}")
 
     def close(self):
-        if self.h:
-            self.lib.lh_mlp_destroy(self.h)
-            self.h = ctypes.c_void_p()
+        h, self.h = self.h, None
+        if h:
+            self.lib.lh_mlp_destroy(h)
 
     def __del__(self):
         try:

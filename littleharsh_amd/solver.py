@@ -50,9 +50,10 @@ class Channel:
     def close(self):
         """Destroy the handle (a batch holding it must be closed first: lh_destroy refuses,
         and the handle then stays alive)."""
-        if getattr(self, "_h", None):
-            if self._lib.lh_destroy(self._h) == capi.LH_OK:
-                self._h = None
+        # at interpreter exit the module's globals may be gone: none is used once lh_destroy has run
+        h, self._h = getattr(self, "_h", None), None
+        if h and self._lib.lh_destroy(h) != 0:
+            self._h = h
 
     def __del__(self):
         self.close()
@@ -242,9 +243,9 @@ class Batch:
                           f"(status {r})", r)
 
     def close(self):
-        if getattr(self, "_b", None):
-            self._lib.lh_batch_destroy(self._b)
-            self._b = None
+        b, self._b = getattr(self, "_b", None), None
+        if b:
+            self._lib.lh_batch_destroy(b)
 
     def __del__(self):
         self.close()
