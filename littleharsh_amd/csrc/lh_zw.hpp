@@ -111,7 +111,9 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) k
   const bool ld_ok = g * zw::COLS + (ev & 7) < mx;      // columns past the plane are not loaded
   // CH / 8 wave-wide loads of 16 bytes per lane into the LDS at m0 + 16 lane.  As asm, because the
   // compiler makes every later LDS read wait for them (it cannot tell the two tile images apart);
-  // the loop waits for them itself, ahead of the barrier that hands the tile over.
+  // the loop waits for them itself, ahead of the barrier that hands the tile over.  Nor does it put wait
+  // states into asm: the load reads M0 one state after its write at the earliest, and the scalar
+  // registers of its base five after a vector instruction's (v_readlane's).  s_mov and s_nop are five.
   const unsigned lds0 = (unsigned)(unsigned long long)(__attribute__((address_space(3))) char*)smem_raw +
                         (unsigned)wv * zw::CHB;
   auto issue = [&](int q, int l, int buf) {
@@ -119,7 +121,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) k
     if (ld_ok) {
 #pragma unroll
       for (int j = 0; j < S::CH / 8; ++j)
-        asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2 nt"
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2 nt"
                      :
                      : "s"(__builtin_amdgcn_readfirstlane(lds0 + (unsigned)buf * S::BUFB + (unsigned)j * (8 * zw::CHB))),
                        "v"(src), "s"(tile.b + j * 8192)
