@@ -12,6 +12,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <map>
 #include <mutex>
 #include <system_error>
 #include <thread>
@@ -61,17 +62,26 @@ __global__ void __launch_bounds__(kXT * 8) k_xfer(XferFields fs, char* stage, in
   }
 }
 
-// The pinned memory, shared by every handle of the process and freed with the last one: the
-// transfer buffers, allocated with the first transfer and used by one transfer at a time (PCIe is
-// the limit of concurrent ones too), and 128-byte slots, one per handle, cut from 32 KB slabs (an
-// allocation per handle costs 0.3 ms).
+// The pinned memory, shared by every handle of the process and freed with the last one: per device
+// the transfer buffers, allocated with its first transfer and used by one transfer at a time (its link
+// to the host is the limit of concurrent ones too), and 128-byte slots, one per handle, cut from 32 KB
+// slabs (an allocation per handle costs 0.3 ms).  A transfer holds its device's lock alone: handles come
+// and go, and other devices transfer, while it waits.
 struct HostStage {
   static constexpr size_t kChunk = 2u << 20;
   static constexpr int kThreads = 4, kSlot = 16, kSlab = 256;    // doubles per slot, slots per slab
-  std::mutex mu;
+  struct Link {
+    std::mutex mu;
+    char* buf = nullptr;
+  };
+  std::mutex mu;                          // of the members below
   int users = 0;
-  char* buf = nullptr;
+  std::map<int, Link> links;              // by device (an entry stays where it is)
   std::vector<double*> slabs, free_slots;
+  Link& link(int dev) {
+    std::lock_guard<std::mutex> g(mu);
+    return links[dev];
+  }
   // a slot for a new handle (null: no pinned memory)
   double* retain() {
     std::lock_guard<std::mutex> g(mu);
@@ -96,8 +106,10 @@ struct HostStage {
     for (double* s : slabs) (void)hipHostFree(s);
     slabs.clear();
     free_slots.clear();
-    if (buf) (void)hipHostFree(buf);
-    buf = nullptr;
+    for (auto& l : links) {               // (no handle is left, so no transfer)
+      if (l.second.buf) (void)hipHostFree(l.second.buf);
+      l.second.buf = nullptr;
+    }
   }
 };
 inline HostStage& host_stage() {
@@ -109,7 +121,7 @@ inline HostStage& host_stage() {
 // in order on stream st of device dev; complete at return
 inline hipError_t xfer_bytes(bool up, int dev, hipStream_t st, char* stage, const XferFields& fs, int nf, int ncol,
                              size_t el) {
-  HostStage& hs = host_stage();
+  HostStage::Link& hs = host_stage().link(dev);
   std::lock_guard<std::mutex> g(hs.mu);
   if (!hs.buf) {
     const hipError_t e = hipHostMalloc((void**)&hs.buf, HostStage::kChunk * HostStage::kThreads, hipHostMallocPortable);
