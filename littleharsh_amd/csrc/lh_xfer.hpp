@@ -112,9 +112,10 @@ struct HostStage {
     }
   }
 };
+// (never destroyed: a host's own global may give its handle back after the statics made later are gone)
 inline HostStage& host_stage() {
-  static HostStage s;
-  return s;
+  static HostStage* const s = new HostStage;
+  return *s;
 }
 
 // the staged bytes of nf fields (element size el, ncol columns) to or from the callers' arrays,
