@@ -211,11 +211,14 @@ int lh_get_launch(lh_handle* h, int* xraw_lc, int* zasm_lc, int* col_bs);
  *   144     12 x 12, 12                         9 x 16, 16
  * xplan selects the plan of the x transforms (length px), zplan that of the z transforms
  * (length pz).  The plans agree to rounding (not bit for bit).  lh_get_plans also returns
- * how many plans each length has (xcount, zcount; 1 or 2). */
+ * how many plans each length has (xcount, zcount; 1 or 2).  The x plan is that of the nonlinear
+ * term in mixed precision and of the canopy; the FP64 nonlinear term, and the canopy of an FP64
+ * channel whose lengths are both at most 144, have radices of their own and do not read it. */
 int lh_set_plans(lh_handle* h, int xplan, int zplan);
 int lh_get_plans(lh_handle* h, int* xplan, int* zplan, int* xcount, int* zcount);
 
-/* lh_autotune first times every (xplan, zplan) pair, then the launch parameters. */
+/* lh_autotune first times every (xplan, zplan) pair, then the launch parameters.  An x plan
+ * that the channel's step does not read stays as it is. */
 int lh_autotune(lh_handle* h, int steps);
 
 /* Many independent channels (handles of any sizes on one device) advanced together: one

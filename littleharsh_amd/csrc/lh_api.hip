@@ -854,6 +854,11 @@ static bool ib_jobs(const lh_handle* h) { return small_channel(h) && h->nibent >
 // The planes of such a channel in FP64 run whole, one block each.  (Mixed precision keeps the three
 // kernels and their order of operations: its results follow every rounding of the canopy rhs.)
 static bool ib_plane(const lh_handle* h) { return ib_jobs(h) && h->prec == LH_PREC_FP64; }
+// whether a kernel of the step reads the x plan: the mixed-precision x pass, and the canopy x pass
+// (k_xs and k_ib_plane have radices of their own)
+static bool xplan_in_step(const lh_handle* h) {
+  return h->prec == LH_PREC_MIXED || (h->nibent > 0 && !ib_plane(h));
+}
 #define LH_IBP_ROW(px, pz, F, ...)             \
   switch (pz) {                                \
     case 48: F<px, 48>(__VA_ARGS__); break;    \
@@ -1901,7 +1906,7 @@ int lh_get_plans(lh_handle* h, int* xplan, int* zplan, int* xcount, int* zcount)
   return LH_OK;
 }
 
-// Search over the FFT plans (every x/z pair), then coordinate search over the launch
+// Search over the FFT plans (every x/z pair that differs), then coordinate search over the launch
 // parameters: every candidate runs `steps` CFL steps (after one warm-up step) timed with
 // events on the handle's stream; the state, the nonlinear terms and the device scalars
 // are saved first and restored afterwards.
@@ -1940,14 +1945,15 @@ int lh_autotune(lh_handle* h, int steps) {
     return LH_OK;
   };
   int r = LH_OK;
-  // every pair of FFT plans (at most 2 x 2), the current pair first
+  // every pair of FFT plans (at most 2 x 2), the current pair first; an x plan that the step does not
+  // read stays as it is
   {
-    const int nxp = plans_of_len(dm.px), nzp = plans_of_len(dm.pz);
+    const int npx = plans_of_len(dm.px), nxp = xplan_in_step(h) ? npx : 1, nzp = plans_of_len(dm.pz);
     const int x00 = h->xplan, z00 = h->zplan;
     int bx = x00, bz = z00;
     float best_ms = 1e30f;
     for (int c = 0; c < nxp * nzp && r == LH_OK; ++c) {
-      h->xplan = (x00 + c / nzp) % nxp;
+      h->xplan = (x00 + c / nzp) % npx;
       h->zplan = (z00 + c % nzp) % nzp;
       if (refresh_ib(h) != hipSuccess) { r = fail(h, LH_ERR_HIP, "lh_autotune: job table"); break; }
       float ms = 0.f;

@@ -198,7 +198,7 @@ class Channel:
         return dict(xplan=v[0].value, zplan=v[1].value, xcount=v[2].value, zcount=v[3].value)
 
     def autotune(self, steps: int = 2):
-        """Times every pair of FFT plans, then the launch parameters; returns the choice."""
+        """Times every pair of FFT plans that the step reads, then the launch parameters; returns the choice."""
         self._chk(self._lib.lh_autotune(self._h, int(steps)), "lh_autotune")
         p = self.get_plans()
         return dict(self.get_launch(), xplan=p["xplan"], zplan=p["zplan"])
