@@ -226,9 +226,9 @@ int lh_autotune(lh_handle* h, int steps);
  * the reference; the instances share nothing).  Per substep, the nonlinear stages of the
  * instances are parallel branches, each on its handle's stream (with the canopy stage of
  * instances whose x or z length exceeds 144); after them the canopy stage of the other
- * instances is one launch per kernel and (length, FFT plan) group, and the column stage
- * (LU of the velocity matrices, velocity sweeps, pressure step) of all instances one launch
- * of each kernel.  A member computes exactly what it computes stepped alone.  After the
+ * instances is one launch for their rhs and one per pair of lengths (in mixed precision one per
+ * kernel and (length, FFT plan) group), and the column stage of all instances one launch of
+ * each kernel in use.  A member computes exactly what it computes stepped alone.  After the
  * step every member's scalars are checked as by lh_step_cfl; the error names the first
  * member that failed. */
 /* A batch re-captures its graph when the CFL number changes or when any member's own graphs

@@ -324,10 +324,12 @@ static void launch_xraw_t(lh_handle* h, const XRAW& a, const void* tw) {
 #endif
 template <typename TR> struct XwWaves { static constexpr int value = sizeof(TR) == 8 ? 8 : LH_XW_WAVES32; };
 static bool use_xw(const lh_handle* h) { return h->dm.px == 576; }
-// products in tiles and the one-wave-per-line z assembly: square FP64 planes of 384 or 576 points,
-// whose z lines fill a wave (per substep, x pass and assembly: 384 x 289 x 384 2.09 ms, with rows and
-// k_zasm 2.77; 256 x 97 x 256 0.36 against 0.49).  Shorter lines leave k_zasm's shape: 96 x 145 x 96
-// reads 0.1 GB in 36 us.  Mixed precision keeps k_zasm's operation order
+// products in tiles and the one-wave-per-line z assembly: FP64 planes whose z lines fill a wave, 384 or
+// 576 points (per substep, x pass and assembly: 384 x 289 x 384 2.09 ms, with rows and k_zasm 2.77;
+// 256 x 97 x 256 0.36 against 0.49), and as long in x, which the x pass's tiles are laid out for (the
+// pairs and group strides of a tile are compiled in); 576 x 384 points and the reverse keep rows and
+// k_zasm.  Shorter lines leave k_zasm's shape: 96 x 145 x 96 reads 0.1 GB in 36 us.  Mixed precision
+// keeps k_zasm's operation order
 static bool use_zw(const lh_handle* h) {
   return h->prec == LH_PREC_FP64 && h->dm.px == h->dm.pz && (h->dm.pz == 576 || h->dm.pz == 384);
 }

@@ -41,7 +41,7 @@ inline size_t colf_lds_bytes(int nyu, int nc, int R, int cb) {
 }
 
 // Rows of a field from a base in scalar registers and a 32-bit byte offset per lane (a field of
-// the largest channel k_col takes holds 0.6 GB)
+// the largest channel k_col takes holds 0.7 GB)
 struct ColF {
   typedef double D2 __attribute__((ext_vector_type(2)));
   char __attribute__((address_space(1)))* b;

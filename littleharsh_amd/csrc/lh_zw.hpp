@@ -8,7 +8,8 @@
 //   Nu2(l) = ikx UV(l) + ikz VW(l) + m_v (VV(l+1) - VV(l))
 // which reads every product row once (one block per field would read nine rows for six) and
 // takes the same six transforms per level.  UV(l) completes Nu1(l) and at once begins Nu1(l+1),
-// so that three sums of 6 values per lane are all a wave carries from product to product (4 values at 384 points).
+// so that three sums of 6 values per lane (4 at 384 points) are all a wave carries from product to
+// product.
 //
 // The x pass writes the products in tiles: the N / 2 row pairs (z, z + N / 2) of 8 kx columns of one
 // product and level are one contiguous run of N / 2 x 16 values, row pair p holding P[k] and P[N
@@ -16,8 +17,8 @@
 // column group and a chunk of levels and takes one tile after the other: the next tile streams
 // from HBM straight into one half of the LDS (global_load_lds, no registers) while the waves
 // transform the tile in the other half, wave w column w, without a barrier among them, with the lanes
-// and radices of the x pass (lh_xw.hpp, lh_xs.hpp) and the column's own
-// places in the tile as its transpose line.  One barrier per tile.
+// and radices of the x pass (lh_xw.hpp, lh_xs.hpp) and the column's own places in the tile as its
+// transpose line.  One barrier per tile, and a second where a finished sum leaves.
 //
 // LDS image of a tile: chunks of four row pairs (64 values, one wave-wide load) 65 values apart,
 // value e = 8 part + column of pair p at place (e + 2 (p % 4)) % 16 of its 16, which spreads the
